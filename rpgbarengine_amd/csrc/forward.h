@@ -137,9 +137,14 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
       sb.part = sx.part + sa.part_floats;
       HIP_CHECK(hipEventRecord(b.ev_fork, stream));
       HIP_CHECK(hipStreamWaitEvent(b.side, b.ev_fork, 0));
-      k::QGemm(sb, grp[1], gn[1], b.side);
+      // (each plans for the compute units of its share of the rows)
+      int64_t rows[2] = {0, 0};
+      for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < gn[i]; ++j) rows[i] += grp[i][j].w.rows;
+      const int side_cus = std::max<int>(1, static_cast<int>(k::ComputeUnits() * rows[1] / (rows[0] + rows[1])));
+      k::QGemm(sb, grp[1], gn[1], b.side, nullptr, side_cus);
       HIP_CHECK(hipEventRecord(b.ev_join, b.side));
-      k::QGemm(sa, grp[0], gn[0], stream);
+      k::QGemm(sa, grp[0], gn[0], stream, nullptr, std::max(1, k::ComputeUnits() - side_cus));
       HIP_CHECK(hipStreamWaitEvent(stream, b.ev_join, 0));
     } else if (n_grp == 1 && gn[0] == 1 && grp[0][0].y == x && grp[0][0].epi == k::kAdd) {
       k::QGemm(sx, grp[0], 1, stream, &pend);  // a K split's sums stay pending

@@ -67,6 +67,9 @@ void SplitRowsAdd(float* X, int64_t ldx, int M, int K, const float* norm_w, floa
 // The reduce launch of a pending sum, into y (row stride ldy, N columns).
 void ApplyPending(const SplitPending& pend, float* y, int64_t ldy, int N, hipStream_t s);
 
+// Compute units of the current device (queried once per device).
+int ComputeUnits();
+
 struct GemmJob {
   MatRef w;
   float* y = nullptr;
@@ -75,43 +78,46 @@ struct GemmJob {
 };
 // True when W can run on QGemm (K-quants need K a multiple of 256).
 bool QGemmSupports(const MatRef& w);
-void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, SplitPending* defer = nullptr);
+// cus: the compute units the launch may count on (0: all), where another
+// runs beside it.
+void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, SplitPending* defer = nullptr,
+           int cus = 0);
 // (defer: for one kAdd job, a K split's sums are left to the caller -- to
 // SplitRowsAdd or ApplyPending before y is read; defer->ksplit stays 1 when
 // nothing is pending)
 // gate.y[t][r] = silu(gate row r . x_t) * (up row r . x_t) in one launch,
 // the same bits as two QGemm products and SwiGLURows -- except where a tiled
-// launch runs its last round's tiles in K halves (more tiles than compute
-// units, that round at most half full): those rows' sums are the halves'
-// sums added, within the products' row bound. Q4_K gate and up of one shape
-// only, and only where QGemm would not split K; false (nothing launched)
-// otherwise.
+// launch runs its last round's tiles in K parts: those rows' sums are the
+// parts' sums added, within the products' row bound. Gate and up of one type
+// and shape; Q4_K, or any type of the tiled launch where that takes the
+// segment, and only where the 32-token kernel would not split K; false
+// (nothing launched) otherwise.
 bool QGemmSwiGLU(const SplitX& x, const GemmJob& gate, const GemmJob& up, hipStream_t s);
 
 // y[i] = silu(g[i]) * u[i] (reference src/kernels.h:82-92), n elements.
 void SwiGLURows(const float* g, const float* u, float* y, int64_t n, hipStream_t s);
 
-// Tiled Q4_K / Q6_K GEMM (gemm_tiled.hip): 128 tokens x 128 weight rows per
-// workgroup, each step's weights unpacked once into LDS. QGemm and QGemmSwiGLU
-// take it for segments of at least kTiledMinTokens tokens.
+// Tiled GEMM (gemm_tiled.hip; Q4_K, Q6_K, Q8_0): 128 tokens x 256 weight rows
+// per workgroup. QGemm and QGemmSwiGLU take it for segments of at least
+// kTiledMinTokens tokens.
 constexpr int kTiledTokens = 128;
-constexpr int kTiledRows = 128;
+constexpr int kTiledRows = 256;
 constexpr int kTiledMinTokens = 96;
 
 struct TiledArgs {
   SplitX x;
   GemmJob job[3];
-  int32_t tiles[3];  // 128-row tiles per job (pair: 64-row tiles of gate and up)
+  int32_t tiles[3];  // 256-row tiles per job (pair: 128-row tiles of gate and up)
   int32_t n_jobs;
   int32_t tiles_m;   // 128-token tiles; workgroup i takes token tile i % tiles_m
   int32_t ksplit;    // blockIdx.y takes super-blocks [y * n / ksplit, (y + 1) * n / ksplit)
   int64_t part_ld;   // partials: x.part[(z * M + token) * part_ld + pcol[job] + row]
   int32_t pcol[3];
   int32_t pair;      // job 0 gate, job 1 up: y = silu(gate.x) * (up.x), no K split
-  // pair only, 0 = none: workgroups from tail_wg on take the tiles from
-  // tail_wg on in halves (the two super-block halves of each, raw sums to
-  // x.part, kTiledTailFloats per half), finished by a second launch
-  int32_t tail_wg = 0;
+  // pair only, tail_split > 1: the tiles from tail_wg on run as tail_split K
+  // parts each (raw sums to x.part, kTiledTailFloats per part), finished by
+  // a second launch
+  int32_t tail_wg = 0, tail_split = 1;
 };
 constexpr int kTiledTailFloats = kTiledTokens * kTiledRows;
 void LaunchTiled(const TiledArgs& a, hipStream_t s);

@@ -53,7 +53,7 @@ __device__ __forceinline__ uint32_t AsU(H2 v) { return __builtin_bit_cast(uint32
 constexpr int kSplitThreads = 256;      // rows of up to 10240 inputs
 constexpr int kSplitThreadsWide = 1024;  // wider rows, up to 40960 inputs
 constexpr int kSplitChunks = 5;          // 8-input chunks per thread at most
-constexpr int kSplitPendMax = 4;         // pending split-K partials a row may carry
+constexpr int kSplitPendMax = 8;         // pending split-K partials a row may carry
 
 template <int NW>
 __device__ __forceinline__ float BlockMax(float v, float* red) {
@@ -76,11 +76,11 @@ __device__ __forceinline__ double PairSum(const double* r) {
 }
 
 // One workgroup of NT threads per token row; NC 8-input chunks per thread
-// (K <= 8 NT NC). kNorm: RMSNorm with gain norm_w; kPend: the pending
-// split-K partials are added first. The prologue's loads (inputs, gains,
+// (K <= 8 NT NC). kNorm: RMSNorm with gain norm_w; kPend > 0: up to kPend
+// pending split-K partials are added first. The prologue's loads (inputs, gains,
 // partials) carry no branches, so all of them are in flight before the
 // first is used.
-template <int NT, int NC, bool kNorm, bool kPend>
+template <int NT, int NC, bool kNorm, int kPend>
 __global__ __launch_bounds__(NT) void SplitRowsKernel(float* X, int64_t ldx, int K, const float* __restrict__ norm_w,
                                                       float eps, SplitX o, SplitPending pend) {
   constexpr int NW = NT / 64;
@@ -110,22 +110,22 @@ __global__ __launch_bounds__(NT) void SplitRowsKernel(float* X, int64_t ldx, int
       wv[c][4] = b.x, wv[c][5] = b.y, wv[c][6] = b.z, wv[c][7] = b.w;
     }
   }
-  if constexpr (kPend) {
+  if constexpr (kPend > 0) {
     // x += the sum of the split partials in split order (SplitKReduceKernel's
     // arithmetic), written back as the residual. Every partial of a chunk
     // (of every chunk, up to two per thread) is requested before any is
     // added: one round trip, not one per split. Split z >= ksplit reloads the
     // last one (an address in bounds) and is not added.
-    constexpr int kGroup = NC <= 2 ? NC : 1;  // chunks whose partials are in flight together
+    constexpr int kGroup = NC * kPend <= 8 ? NC : 1;  // chunks whose partials are in flight together
     const int nz = pend.ksplit;
 #pragma unroll
     for (int c0 = 0; c0 < NC; c0 += kGroup) {
-      float4 pp[kGroup][kSplitPendMax][2];
+      float4 pp[kGroup][kPend][2];
 #pragma unroll
       for (int g = 0; g < kGroup; ++g) {
         const int ch = min(tid + (c0 + g) * NT, n8 - 1);
 #pragma unroll
-        for (int z = 0; z < kSplitPendMax; ++z) {
+        for (int z = 0; z < kPend; ++z) {
           const int zz = min(z, nz - 1);
           const float4* p4 = reinterpret_cast<const float4*>(
               pend.part + (static_cast<int64_t>(zz) * pend.M + t) * pend.part_ld + pend.pcol + 8 * ch);
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(NT) void SplitRowsKernel(float* X, int64_t ldx, int
         const int c = c0 + g, ch = tid + c * NT;
         float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int z = 0; z < kSplitPendMax; ++z) {
+        for (int z = 0; z < kPend; ++z) {
           if (z == 0 || z < nz) {  // nz >= 1
             const float4 a = pp[g][z][0], b = pp[g][z][1];
             sum[0] += a.x, sum[1] += a.y, sum[2] += a.z, sum[3] += a.w;
@@ -232,7 +232,8 @@ constexpr int kStep = 64;            // inputs per pipeline step
 constexpr int kARow = kStep + 8;     // LDS row of one token's step (f16, padded)
 
 constexpr int kGemmSplitMax = 4;     // K splits of one product (partials summed in order)
-static_assert(kGemmSplitMax <= kSplitPendMax, "SplitRows holds every pending partial of a chunk in flight");
+constexpr int kTiledSplitMax = 8;    // those of a tiled launch
+static_assert(kGemmSplitMax <= kTiledSplitMax && kTiledSplitMax <= kSplitPendMax, "SplitRows holds every pending partial of a chunk in flight");
 
 struct GemmArgs {
   SplitX x;
@@ -986,11 +987,22 @@ void SwiGLURows(const float* g, const float* u, float* y, int64_t n, hipStream_t
   HIP_CHECK(hipGetLastError());
 }
 
+namespace {
+// Floats of the split-K partials. Tiled launches (kTiledMinTokens tokens and
+// more) run at most kTiledPartTiles partial tiles, whatever M; the 32-token
+// kernels split at most kGemmSplitMax ways.
+constexpr int64_t kTiledPartTiles = 512;
+int64_t PartFloats(int M, int n_max) {
+  return M >= kTiledMinTokens ? kTiledPartTiles * kTiledTailFloats
+                              : static_cast<int64_t>(kGemmSplitMax) * M * n_max;
+}
+}  // namespace
+
 size_t SplitXBytes(int M, int K, int n_max) {
   const size_t big = static_cast<size_t>(M) * K * 2, small = static_cast<size_t>(M) * (K / 32) * 2;
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   return 2 * up(big) + 2 * up(small) + up(static_cast<size_t>(M) * 4) +
-         up(static_cast<size_t>(kGemmSplitMax) * M * n_max * 4);
+         up(static_cast<size_t>(PartFloats(M, n_max)) * 4);
 }
 
 SplitX SplitXView(void* base, int M, int K, int n_max) {
@@ -1004,7 +1016,7 @@ SplitX SplitXView(void* base, int M, int K, int n_max) {
   s.sum_lo = p + 2 * up(big) + up(small);
   s.inv_s = reinterpret_cast<float*>(p + 2 * up(big) + 2 * up(small));
   s.part = reinterpret_cast<float*>(p + 2 * up(big) + 2 * up(small) + up(static_cast<size_t>(M) * 4));
-  s.part_floats = static_cast<int64_t>(kGemmSplitMax) * M * n_max;
+  s.part_floats = PartFloats(M, n_max);
   s.M = M;
   s.K = K;
   return s;
@@ -1024,15 +1036,19 @@ void SplitRowsAdd(float* X, int64_t ldx, int M, int K, const float* norm_w, floa
   const bool wide = K > 8 * kSplitChunks * kSplitThreads;
   const int nt = wide ? kSplitThreadsWide : kSplitThreads;
   const int nc = static_cast<int>(CeilDiv(K / 8, nt));
-  const int variant = (norm_w != nullptr ? 1 : 0) | (pend.part != nullptr ? 2 : 0);
+  const int variant =
+      (norm_w != nullptr ? 1 : 0) + (pend.part == nullptr ? 0 : pend.ksplit <= kGemmSplitMax ? 2 : 4);
   auto launch = [&](auto nt_c, auto nc_c) {
     constexpr int NT = decltype(nt_c)::value, NC = decltype(nc_c)::value;
+    constexpr int P4 = kGemmSplitMax, P8 = kSplitPendMax;
     const dim3 block(NT);
     switch (variant) {
-      case 0: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, false, false>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend); break;
-      case 1: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, true, false>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend); break;
-      case 2: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, false, true>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend); break;
-      default: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, true, true>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend);
+      case 0: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, false, 0>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend); break;
+      case 1: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, true, 0>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend); break;
+      case 2: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, false, P4>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend); break;
+      case 3: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, true, P4>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend); break;
+      case 4: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, false, P8>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend); break;
+      default: hipLaunchKernelGGL((SplitRowsKernel<NT, NC, true, P8>), grid, block, 0, s, X, ldx, K, norm_w, eps, o, pend);
     }
   };
   using N256 = std::integral_constant<int, kSplitThreads>;
@@ -1067,6 +1083,19 @@ bool QGemmSupports(const MatRef& w) {
   return ((w.type == kQ4_K || w.type == kQ6_K) && w.cols % 256 == 0) || (w.type == kQ8_0 && w.cols % 64 == 0);
 }
 
+int ComputeUnits() {
+  static int cached[64] = {};
+  int dev = 0;
+  HIP_CHECK(hipGetDevice(&dev));
+  RPG_CHECK(dev >= 0 && dev < 64, "device %d", dev);
+  if (cached[dev] == 0) {
+    int n = 0;
+    HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+    cached[dev] = n > 0 ? n : 1;
+  }
+  return cached[dev];
+}
+
 namespace {
 
 // y = (y +) the sum of the split-K partials of one job, in split order.
@@ -1078,13 +1107,13 @@ __global__ __launch_bounds__(256) void SplitKReduceKernel(const float* __restric
   // every partial (and y) requested before the first is added: one round trip
   float* yp = y + static_cast<int64_t>(tok) * ldy + row;
   const float y0 = epi == kAdd ? *yp : 0.0f;
-  float p[kGemmSplitMax];
+  float p[kTiledSplitMax];
 #pragma unroll
-  for (int z = 0; z < kGemmSplitMax; ++z)
+  for (int z = 0; z < kTiledSplitMax; ++z)
     if (z < ksplit) p[z] = part[(static_cast<int64_t>(z) * M + tok) * part_ld + pcol + row];
   float v = 0.0f;
 #pragma unroll
-  for (int z = 0; z < kGemmSplitMax; ++z)
+  for (int z = 0; z < kTiledSplitMax; ++z)
     if (z < ksplit) v += p[z];
   *yp = epi == kAdd ? y0 + v : v;
 }
@@ -1101,37 +1130,33 @@ int ChooseSplit(int64_t wgs, int nblk, int64_t cols, const SplitX& x, int64_t ta
   return S;
 }
 
-// Compute units of the current device (queried once per device).
-int ComputeUnits() {
-  static int cached[64] = {};
-  int dev = 0;
-  HIP_CHECK(hipGetDevice(&dev));
-  RPG_CHECK(dev >= 0 && dev < 64, "device %d", dev);
-  if (cached[dev] == 0) {
-    int n = 0;
-    HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
-    cached[dev] = n > 0 ? n : 1;
+// The K parts (1 .. kTiledSplitMax) of `wgs` tiled workgroups of `nblk`
+// super-blocks on `cus` compute units (one tiled workgroup per unit): the
+// count whose rounds of workgroups take the least time, a workgroup costing
+// its super-blocks plus about 1.5 of pipeline fill and output. Every part
+// keeps at least 2.5 super-blocks on average, and at most `max_parts` partial
+// tiles are written.
+int TiledParts(int64_t wgs, int nblk, int64_t cus, int64_t max_parts) {
+  int best = 1;
+  double best_cost = 0.0;
+  for (int c = 1; c <= kTiledSplitMax; ++c) {
+    if (c > 1 && (5 * c > 2 * nblk || c * wgs > max_parts)) break;
+    const double cost = static_cast<double>(CeilDiv(c * wgs, cus)) * (static_cast<double>(nblk) / c + 1.5);
+    if (c == 1 || cost < 0.95 * best_cost) best = c, best_cost = cost;
   }
-  return cached[dev];
+  return best;
 }
 
-// K splits of a tiled launch of `wgs` workgroups over `nblk` super-blocks:
-// the largest S <= kGemmSplitMax whose S * wgs workgroups fit in one round
-// of the compute units (one tiled workgroup per unit), with at least 4
-// super-blocks per split and room for the partials. A launch of 80 tiles on
-// 256 units takes S = 3 (240 workgroups in one round) rather than 4 (320,
-// a second round of 64).
-int TiledSplit(int64_t wgs, int nblk, int64_t cols, const SplitX& x) {
-  const int64_t cus = ComputeUnits();
-  int S = 1;
-  for (int c = 2; c <= kGemmSplitMax; ++c)
-    if (c * wgs <= cus && 4 * c <= nblk && static_cast<int64_t>(c) * x.M * cols <= x.part_floats) S = c;
-  return S;
+// Whether a launch of this matrix over x takes the tiled kernel (its buffer
+// resources and lane offsets are 32-bit).
+bool TiledTakes(const MatRef& w, const SplitX& x) {
+  return x.M >= kTiledMinTokens && (w.type == kQ4_K || w.type == kQ6_K || w.type == kQ8_0) && x.K % 256 == 0 &&
+         w.row_bytes * w.rows < (int64_t{1} << 31) && static_cast<int64_t>(x.M) * x.K * 2 < (int64_t{1} << 31);
 }
 
 }  // namespace
 
-void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, SplitPending* defer) {
+void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, SplitPending* defer, int cus) {
   if (defer != nullptr) *defer = SplitPending{};
   RPG_CHECK(n_jobs >= 1 && n_jobs <= 3, "qgemm: 1..3 jobs");
   int32_t pcol[3] = {0, 0, 0};
@@ -1144,11 +1169,8 @@ void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, Spli
   }
   int S = 1;
   const bool q6 = jobs[0].w.type == kQ6_K;
-  // Q4_K / Q6_K launches of long segments take the tiled kernel. (Its K
-  // split fills at most one round of compute units, so the q,k launch -- 160
-  // workgroups at 512 tokens -- leaves room for the v launch beside it on
-  // the side stream.)
-  if ((jobs[0].w.type == kQ4_K || q6) && x.M >= kTiledMinTokens) {
+  // Launches of long segments take the tiled kernel.
+  if (TiledTakes(jobs[0].w, x)) {
     TiledArgs t;
     t.x = x;
     t.pair = 0;
@@ -1161,7 +1183,9 @@ void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, Spli
       t.pcol[j] = pcol[j];
       tiles += t.tiles[j];
     }
-    S = TiledSplit(static_cast<int64_t>(tiles) * t.tiles_m, x.K / 256, cols, x);
+    S = TiledParts(static_cast<int64_t>(tiles) * t.tiles_m, x.K / 256, cus > 0 ? cus : ComputeUnits(),
+                   x.part_floats / kTiledTailFloats);
+    while (S > 1 && static_cast<int64_t>(S) * x.M * cols > x.part_floats) --S;
     t.ksplit = S;
     t.part_ld = cols;
     LaunchTiled(t, s);
@@ -1229,7 +1253,7 @@ void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, Spli
 
 void ApplyPending(const SplitPending& pend, float* y, int64_t ldy, int N, hipStream_t s) {
   if (pend.part == nullptr) return;
-  RPG_CHECK(pend.ksplit >= 1 && pend.ksplit <= kGemmSplitMax, "pending sums: %d splits", pend.ksplit);
+  RPG_CHECK(pend.ksplit >= 1 && pend.ksplit <= kTiledSplitMax, "pending sums: %d splits", pend.ksplit);
   const int64_t n = static_cast<int64_t>(pend.M) * N;
   hipLaunchKernelGGL(SplitKReduceKernel, dim3(static_cast<unsigned>(CeilDiv(n, 256))), dim3(256), 0, s, pend.part,
                      pend.part_ld, pend.pcol, pend.ksplit, pend.M, N, y, ldy, static_cast<int>(kAdd));
@@ -1237,15 +1261,11 @@ void ApplyPending(const SplitPending& pend, float* y, int64_t ldy, int N, hipStr
 }
 
 bool QGemmSwiGLU(const SplitX& x, const GemmJob& gate, const GemmJob& up, hipStream_t s) {
-  if (gate.w.type != kQ4_K || up.w.type != kQ4_K || gate.w.rows != up.w.rows || gate.w.cols != x.K ||
-      up.w.cols != x.K || gate.w.row_bytes != up.w.row_bytes || x.K % 256 != 0)
+  if (gate.w.type != up.w.type || gate.w.rows != up.w.rows || gate.w.cols != x.K || up.w.cols != x.K ||
+      gate.w.row_bytes != up.w.row_bytes || x.K % 256 != 0)
     return false;
-  if (x.M >= kTiledMinTokens) {
-    // the tiled launch; fused only where the unfused one would not split
+  if (TiledTakes(gate.w, x)) {
     const int64_t mt = CeilDiv(x.M, kTiledTokens);
-    if (TiledSplit(2 * CeilDiv(gate.w.rows, kTiledRows) * mt, x.K / 256, 2 * static_cast<int64_t>(gate.w.rows), x) >
-        1)
-      return false;
     TiledArgs t;
     t.x = x;
     t.pair = 1;
@@ -1258,16 +1278,15 @@ bool QGemmSwiGLU(const SplitX& x, const GemmJob& gate, const GemmJob& up, hipStr
     t.pcol[0] = t.pcol[1] = t.pcol[2] = 0;
     t.ksplit = 1;
     t.part_ld = 0;
-    // More tiles than compute units, with a last round at most half full:
-    // that round's tiles run as two halves each (twice the workgroups at
-    // half the length), their sums added by a second launch.
+    // The tiles past the last full round of compute units run in K parts,
+    // their sums added by a second launch.
     const int64_t total = t.tiles[0] * mt, cus = ComputeUnits(), tail = total % cus;
-    if (total > cus && tail > 0 && 2 * tail <= cus && x.K >= 512 &&
-        tail * 2 * kTiledTailFloats <= x.part_floats)
-      t.tail_wg = static_cast<int32_t>(total - tail);
+    t.tail_wg = static_cast<int32_t>(total - tail);
+    t.tail_split = tail > 0 ? TiledParts(tail, x.K / 256, cus, x.part_floats / kTiledTailFloats) : 1;
     LaunchTiled(t, s);
     return true;
   }
+  if (gate.w.type != kQ4_K) return false;
   using Shape = G4Shape<kG4Mtw, kG4Wm>;
   const int64_t mtiles = CeilDiv(x.M, Shape::kTokens);
   const int tiles = static_cast<int>(CeilDiv(gate.w.rows, kG4Rows / 2));

@@ -137,6 +137,61 @@ def test_tiled_gemm_ragged_shapes(qtype, k, rows, m):
     assert np.all(Y[m - 1] == 0.0)
 
 
+# The tiled kernel's Q8_0 form and its K parts: token and row tiles partly
+# empty, one row, part ranges of unequal length (38 super-blocks in 8).
+@pytest.mark.parametrize("qtype,k,rows,m", [(synth.Q8_0, 2560, 300, 130), (synth.Q8_0, 256, 1, 100),
+                                            (synth.Q8_0, 9728, 257, 129), (synth.Q6_K, 9728, 257, 129),
+                                            (synth.Q4_K, 9728, 513, 97)])
+def test_tiled_gemm_256_rows(qtype, k, rows, m):
+    w32 = synth.gaussian(41, k + rows + qtype, rows * k, 0.02).reshape(rows, k)
+    raw = synth.quantize(qtype, w32)
+    wdq = oracle.dequant(qtype, raw.reshape(-1), rows * k).reshape(rows, k)
+    X = synth.gaussian(43, m + k, m * k, 1.0).reshape(m, k)
+    X[1] *= 3.0e4
+    X[m - 1] = 0.0
+    Y = eng.matmul(qtype, raw, rows, k, X)
+    assert rel_row_error(Y[: m - 1], X[: m - 1], wdq) <= 1e-6
+    assert np.all(Y[m - 1] == 0.0)
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+def test_tiled_gemm_common_error(qtype):
+    """The matrix core rounds its sums down; the tiled kernel's alternating
+    signs cancel that. Inputs with a heavy tail (cubed normals): the mean
+    error over 65536 outputs, each with an error of about 2e-7 of the outputs'
+    root mean square shared by up to 256 tokens of a row, stays below
+    6e-8 (without the signs it measured 1e-7 and more on long chains)."""
+    k, rows, m = 2048, 256, 256
+    w32 = synth.gaussian(51, k + qtype, rows * k, 0.02).reshape(rows, k)
+    raw = synth.quantize(qtype, w32)
+    wdq = oracle.dequant(qtype, raw.reshape(-1), rows * k).reshape(rows, k).astype(np.float64)
+    X = synth.gaussian(53, k, m * k, 1.0).reshape(m, k) ** 3
+    Y = eng.matmul(qtype, raw, rows, k, X)
+    R = X.astype(np.float64) @ wdq.T
+    assert abs(np.mean(Y - R)) <= 6e-8 * np.sqrt(np.mean(R * R))
+
+
+# A fused gate/up/SwiGLU launch whose tiles run in K parts: every tile (one
+# token tile, a partial row tile), and the tiles past a full round of 256
+# compute units (23 x 12 = 276) -- Q4_K and Q8_0.
+@pytest.mark.parametrize("qtype,rows,k,m", [(synth.Q4_K, 1000, 2560, 101), (synth.Q8_0, 1000, 2560, 101),
+                                            (synth.Q4_K, 2820, 2560, 1413)])
+def test_gate_up_swiglu_tail_parts(qtype, rows, k, m):
+    g = synth.quantize(qtype, synth.gaussian(61, rows + k, rows * k, 0.02).reshape(rows, k))
+    u = synth.quantize(qtype, synth.gaussian(62, rows + k, rows * k, 0.02).reshape(rows, k))
+    X = synth.gaussian(63, m, m * k, 1.0).reshape(m, k)
+    Y, fused = eng.matmul_swiglu(qtype, g, u, rows, k, X)
+    assert fused
+    G = eng.matmul(qtype, g, rows, k, X).astype(np.float64)
+    U = eng.matmul(qtype, u, rows, k, X).astype(np.float64)
+    want = G / (1.0 + np.exp(-G)) * U
+    # both sides' sums carry up to 1e-6 of sum|a*w| (the row bound), some
+    # 1e-5 of a sum's own size; most outputs are far closer
+    err = np.abs(Y - want)
+    assert np.sqrt(np.mean(err ** 2)) <= 2e-6 * np.sqrt(np.mean(want ** 2))
+    assert err.max() <= 1e-4 * np.sqrt(np.mean(want ** 2))
+
+
 # one-token shapes: a single super-block, odd super-block counts (Q6_K rows
 # then alternate between 4- and 2-byte alignment), the largest input the
 # matrix-core path stages, one beyond it (the wave kernel takes it), one
