@@ -560,7 +560,9 @@ int32_t rpg_hip_attention(const float* q, const float* k, const float* v, int32_
     RPG_CHECK(seq > 0 && pos0 >= 0 && n_kv > 0 && n_heads > 0 && n_heads % n_kv == 0, "attention: bad shape");
     const int64_t n_pos = static_cast<int64_t>(pos0) + seq;
     const size_t qb = static_cast<size_t>(seq) * n_heads * 128 * 4, cb = static_cast<size_t>(n_kv) * n_pos * 128 * 4;
-    DevBuf dq(qb), dk(cb), dv(cb), dout(qb);
+    // partial states of the most key ranges a launch may take
+    const int64_t part = std::min<int64_t>(32, CeilDiv(n_pos, 64)) * seq * n_heads * 130;
+    DevBuf dq(qb), dk(cb), dv(cb), dout(qb), dpart(static_cast<size_t>(part) * 4);
     HIP_CHECK(hipMemcpy(dq.p, q, qb, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(dk.p, k, cb, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(dv.p, v, cb, hipMemcpyHostToDevice));
@@ -575,6 +577,8 @@ int32_t rpg_hip_attention(const float* q, const float* k, const float* v, int32_
     a.hd = 128;
     a.max_seq = n_pos;
     a.pos0_host = pos0;
+    a.part = dpart.as<float>();
+    a.part_floats = part;
     RPG_CHECK(seq > 1, "attention: the segment kernel takes seq >= 2");
     k::Attention(a, nullptr);
     HIP_CHECK(hipMemcpy(out, dout.p, qb, hipMemcpyDeviceToHost));

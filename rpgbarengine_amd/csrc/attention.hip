@@ -13,11 +13,14 @@
 // RoPE and the cache write folded in, is in decode.hip.)
 //
 // Prefill (several queries): PrefillKernel, workgroup (kv head, 16 or 32
-// queries), two waves per query head of the group splitting the key blocks,
+// queries, and where these leave compute units idle one of several key
+// ranges, merged by MergePrefillKernel), two waves per query head of the group splitting the key blocks,
 // scores and P.V as f16 hi/lo products on the matrix cores (16x16x32), K/V
 // blocks of 32 positions staged once for the group, online softmax.
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "common.h"
 #include "expf_glibc.h"
@@ -33,6 +36,7 @@ namespace {
 constexpr int kChunk = 64;  // positions per decode split
 constexpr int kHd = 128;
 constexpr int kMaxGroup = 8;
+constexpr int kMaxPrefillSplits = 32;  // key ranges of a split prefill attention (at most a wave's lanes)
 
 __device__ __forceinline__ float WaveMax(float v) {
 #pragma unroll
@@ -209,7 +213,10 @@ __device__ __forceinline__ F4v Mfma16x3(H8v ah, H8v al, H8v bh, H8v bl, F4v c) {
 // G: query heads per KV head. Two waves per head split the key blocks (even
 // and odd) and merge their online-softmax states at the end; QT query tiles
 // of 16 share the workgroup's staged K/V blocks (long segments at G <= 2:
-// half the staging per query), so a workgroup has 2 G QT waves.
+// half the staging per query), so a workgroup has 2 G QT waves. With
+// gridDim.z = S > 1, workgroup z takes the z-th of S ranges of the block's
+// key steps and leaves its state to MergePrefillKernel (a.part: the output
+// sums [z][query][head][128], then (m, l) [z][query][head]).
 template <int G, int QT>
 __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   constexpr int nt = 128 * G * QT;
@@ -246,7 +253,20 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   const float* kb = a.kcache + static_cast<int64_t>(kh) * a.max_seq * kHd;
   const float* vb = a.vcache + static_cast<int64_t>(kh) * a.max_seq * kHd;
   const int n_blocks = (n_keys + kKB - 1) / kKB;
-  const int n_steps = (n_blocks + kBS - 1) / kBS;
+  const int n_steps_all = (n_blocks + kBS - 1) / kBS;
+  const int n_split = static_cast<int>(gridDim.z), z = static_cast<int>(blockIdx.z);
+  const int st0 = z * n_steps_all / n_split, n_steps = (z + 1) * n_steps_all / n_split;
+  float2* const part_ml =
+      reinterpret_cast<float2*>(a.part + static_cast<int64_t>(n_split) * a.seq * a.n_heads * kHd);
+  if (st0 == n_steps) {
+    // more ranges than steps: an empty state
+    for (int i = tid; i < kQB * QT * G; i += nt) {
+      const int t = t0b + i / G;
+      if (t < a.seq)
+        part_ml[(static_cast<int64_t>(z) * a.seq + t) * a.n_heads + kh * G + i % G] = float2{-__builtin_inff(), 0.0f};
+    }
+    return;
+  }
   // step i stages blocks kBS i .. kBS i + kBS - 1: K as float4 units u = block
   // (u / 1024), key ((u / 32) % 32), column (u % 32) (32 lanes read one key
   // row and write it contiguously); V as units of 4 keys x
@@ -278,7 +298,7 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
       }
     }
   };
-  load_step(0);
+  load_step(st0);
   // (after the first K/V loads, so that both round trips overlap)
   // this lane's query row c16 (clamped past the segment: computed, not
   // stored), dimensions 32 c + 8 kg .. + 7 of chunk c, split hi + lo
@@ -309,7 +329,7 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) SplitHalf(x[c][i] * sq, qh[c], ql[c], i);
   }
-  for (int st = 0; st < n_steps; ++st) {
+  for (int st = st0; st < n_steps; ++st) {
     __syncthreads();  // the previous step's LDS reads are done
 #pragma unroll
     for (int i = 0; i < kKPer; ++i) {
@@ -446,8 +466,11 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   if (half == 0) {
     const float m1 = xm[lane * 2], l1 = xm[lane * 2 + 1];
     const float mn = fmaxf(m, m1);
-    f0 = ExpSoft(m - mn);
-    f1 = ExpSoft(m1 - mn);
+    // (a range of keys past this query has seen none: m = -inf, l = 0)
+    const bool none = mn == -__builtin_inff();
+    f0 = none ? 0.0f : ExpSoft(m - mn);
+    f1 = none ? 0.0f : ExpSoft(m1 - mn);
+    m = mn;
     l = __builtin_fmaf(l, f0, l1 * f1);
   }
   float* xo = kvf + QT * G * 64 * 2 + (qt * G + hg) * 64 * 16;  // [lane][4 tiles x 4 dimensions]
@@ -471,10 +494,70 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   if (half != 0) return;
   const int t = t0 + c16;
   if (t >= a.seq) return;
+  if (n_split > 1) {
+    const int64_t row = (static_cast<int64_t>(z) * a.seq + t) * a.n_heads + h;
+    float* po = a.part + row * kHd + 4 * kg;
+#pragma unroll
+    for (int ct = 0; ct < 8; ++ct) *reinterpret_cast<F4v*>(po + 16 * ct) = o[ct];
+    if (kg == 0) part_ml[row] = float2{m, l};
+    return;
+  }
   float* out = a.out + (static_cast<int64_t>(t) * a.n_heads + h) * kHd + 4 * kg;
 #pragma unroll
   for (int ct = 0; ct < 8; ++ct)
     *reinterpret_cast<float4*>(out + 16 * ct) = make_float4(o[ct][0] / l, o[ct][1] / l, o[ct][2] / l, o[ct][3] / l);
+}
+
+// The split prefill attention's output: one wave per (query, head) adds its
+// S states, each rescaled by exp(m_z - max m), and divides by the summed l;
+// lane d takes dimensions 2 d and 2 d + 1. A state that saw no key (l = 0) is
+// not read: its sums may be unwritten.
+__global__ __launch_bounds__(256) void MergePrefillKernel(AttnArgs a, int n_split) {
+  const int64_t rows = static_cast<int64_t>(a.seq) * a.n_heads;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= rows) return;
+  const float2* ml = reinterpret_cast<const float2*>(a.part + n_split * rows * kHd);
+  float m = -__builtin_inff(), l = 0.0f;
+  if (lane < n_split) {
+    const float2 v = ml[lane * rows + row];
+    m = v.x, l = v.y;
+  }
+  const float mx = WaveMax(m);  // (finite: every query sees key 0)
+  const float f = l > 0.0f ? ExpSoft(m - mx) : 0.0f;
+  const float total = WaveSum(l * f);
+  const float2* po = reinterpret_cast<const float2*>(a.part + row * kHd) + lane;
+  float ox = 0.0f, oy = 0.0f;
+  for (int z0 = 0; z0 < n_split; z0 += 4) {
+    float2 v[4];
+    float fz[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int z = z0 + i;
+      fz[i] = z < n_split ? __shfl(f, z, 64) : 0.0f;  // (uniform)
+      v[i] = float2{0.0f, 0.0f};
+      if (fz[i] != 0.0f) v[i] = po[z * rows * (kHd / 2)];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      ox = __builtin_fmaf(v[i].x, fz[i], ox);
+      oy = __builtin_fmaf(v[i].y, fz[i], oy);
+    }
+  }
+  reinterpret_cast<float2*>(a.out + row * kHd)[lane] = float2{ox / total, oy / total};
+}
+
+// Key ranges of a prefill attention of `wgs` workgroups whose longest query
+// block walks `steps` steps of 64 keys: enough ranges for about two
+// workgroups per compute unit (their LDS lets two share one), at most one per
+// step and at most what the partials' buffer holds. Two ranges do not pay for
+// the merge (512 tokens of the 4B shape: 31 + 7.5 us against 37); from three
+// on they do: 203 queries behind 1500 keys (104 workgroups, 4 ranges) 106 ->
+// 60 + 6 us, 37 behind 611 (24 workgroups, 11 ranges) 45.6 -> 17.8 + 4.8 us.
+int PrefillSplits(int64_t wgs, int64_t steps, int64_t part_floats, int64_t row_floats) {
+  const int64_t room = part_floats / row_floats;
+  const int64_t s = std::min<int64_t>({kMaxPrefillSplits, 512 / std::max<int64_t>(wgs, 1), steps, room});
+  return s < 3 ? 1 : static_cast<int>(s);
 }
 
 }  // namespace
@@ -495,7 +578,11 @@ void Attention(const AttnArgs& a, hipStream_t s) {
     RPG_CHECK(a.pos0_dev == nullptr, "prefill attention takes a host position");
     const int64_t n_keys_max = static_cast<int64_t>(a.pos0_host) + a.seq;
     RPG_CHECK(a.pos0_host >= 0 && n_keys_max <= a.max_seq, "attention past the cache capacity");
-    const dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(CeilDiv(a.seq, kQB)));
+    const int64_t q_blocks = CeilDiv(a.seq, kQB);
+    const int splits =
+        PrefillSplits(a.n_kv * q_blocks, CeilDiv(n_keys_max, 2 * kKB), a.part != nullptr ? a.part_floats : 0,
+                      static_cast<int64_t>(a.seq) * a.n_heads * (kHd + 2));
+    const dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(q_blocks), static_cast<unsigned>(splits));
     // long segments at G <= 2: two query tiles per workgroup (half the
     // workgroups, each staged K/V block read by twice the queries)
     const bool wide = a.seq >= kWideQueries && CeilDiv(a.seq, 2 * kQB) * a.n_kv >= 256;
@@ -519,6 +606,11 @@ void Attention(const AttnArgs& a, hipStream_t s) {
       case 6: hipLaunchKernelGGL((PrefillKernel<6, 1>), grid, dim3(768), 0, s, a); break;
       case 7: hipLaunchKernelGGL((PrefillKernel<7, 1>), grid, dim3(896), 0, s, a); break;
       default: hipLaunchKernelGGL((PrefillKernel<8, 1>), grid, dim3(1024), 0, s, a); break;
+    }
+    if (!wide && splits > 1) {
+      HIP_CHECK(hipGetLastError());
+      const int64_t rows = static_cast<int64_t>(a.seq) * a.n_heads;
+      hipLaunchKernelGGL(MergePrefillKernel, dim3(static_cast<unsigned>(CeilDiv(rows, 4))), dim3(256), 0, s, a, splits);
     }
   }
   HIP_CHECK(hipGetLastError());

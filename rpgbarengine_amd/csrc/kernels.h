@@ -95,6 +95,11 @@ struct AttnArgs {
   int64_t max_seq;
   const int32_t* pos0_dev;
   int32_t pos0_host;
+  // partial states of several queries' attention, for splitting their keys
+  // over workgroups where the queries alone leave compute units idle; it may
+  // be null (no split)
+  float* part = nullptr;
+  int64_t part_floats = 0;
 };
 int64_t AttnWorkFloats(int n_heads, int64_t max_seq);
 void Attention(const AttnArgs& a, hipStream_t s);

@@ -22,6 +22,10 @@ constexpr int64_t kPrefillChunk = 4096;
 // Tokens per pass when every position's logits are returned (the logits
 // buffer holds a row per token of the pass, 0.6 MB each).
 constexpr int64_t kLogitRowsChunk = 512;
+// Least size of the operand buffer, whose room between projections holds the
+// partial states of a short segment's attention (37 tokens of the 4B shape
+// in 26 key ranges).
+constexpr size_t kAttnPartBytes = size_t{16} << 20;
 constexpr int kGenChunk = 16;           // decode steps between host stop checks
 // The persistent decode step needs every one of its workgroups resident at
 // once; two of them running together (sessions generating from different
@@ -248,6 +252,7 @@ void Session::EnsureScratch(int64_t tokens, int64_t logit_rows) {
   }
   if (split_) HIP_CHECK(hipFree(split_));
   split_ = nullptr;
+  split_bytes_ = 0;
   auto alloc = [&](float** p, int64_t per_token) {
     DeviceAlloc(p, sizeof(float) * static_cast<size_t>(tokens * per_token));
   };
@@ -262,7 +267,10 @@ void Session::EnsureScratch(int64_t tokens, int64_t logit_rows) {
   if (tokens >= 2) {  // GEMM operands of multi-token segments
     alloc(&gu_, 2 * static_cast<int64_t>(c.intermediate));
     const int kmax = std::max({c.hidden, c.q_dim(), c.intermediate});
-    DeviceAlloc(&split_, k::SplitXBytes(static_cast<int>(tokens), kmax, SplitColumns(c)));
+    const size_t split_bytes =
+        std::max(k::SplitXBytes(static_cast<int>(tokens), kmax, SplitColumns(c)), kAttnPartBytes);
+    DeviceAlloc(&split_, split_bytes);
+    split_bytes_ = static_cast<int64_t>(split_bytes);
   }
   scratch_tokens_ = tokens;
   logit_rows_cap_ = logit_rows;
@@ -322,6 +330,9 @@ void Session::ForwardSegment(const int32_t* ids_dev, int64_t n, int64_t pos0, co
     aa.max_seq = max_seq_;
     aa.pos0_dev = pos_dev;
     aa.pos0_host = static_cast<int32_t>(pos0);
+    // (the GEMMs' operand buffer is idle between the QKV and O projections)
+    aa.part = static_cast<float*>(split_);
+    aa.part_floats = split_ ? split_bytes_ / 4 : 0;
     k::Attention(aa, stream_);
   });
   if (logit_rows == 1 && m_.lm_head_tiled().w != nullptr) {
