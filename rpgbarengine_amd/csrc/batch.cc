@@ -97,7 +97,10 @@ void SessionBatch::EnqueueStep(bool forced) {
   if (forced) k::ForceTokens(d_tok_, B_, d_force_, d_drawn_, d_step_, out_cap_, stream_);
   k::GatherRows(m_.embd(), d_tok_, B_, x_, H, d_err_, stream_, d_out_, d_step_, out_cap_);
   const FwdBufs b{x_, h_, q_, k_, v_, attn_, act_, gu_, split_, SplitColumns(c), stream_, side_, ev_fork_, ev_join_};
-  ForwardLayers(m_, b, B_, [&](int l, const LayerDev& w) {
+  ForwardLayers(m_, b, B_, [&](int l, const LayerDev& w, const k::SplitPending* pend) {
+    k::ApplyPending(pend[0], q_, c.q_dim(), c.q_dim(), stream_, k::kStore);
+    k::ApplyPending(pend[1], k_, c.kv_dim(), c.kv_dim(), stream_, k::kStore);
+    k::ApplyPending(pend[2], v_, c.kv_dim(), c.kv_dim(), stream_, k::kStore);
     k::DecodeAttnBatchArgs ab{};
     ab.base.q = q_;
     ab.base.k = k_;

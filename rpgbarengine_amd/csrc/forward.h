@@ -37,8 +37,9 @@ struct FwdBufs {
 inline int SplitColumns(const ModelConfig& c) { return std::max(c.hidden, c.q_dim() + 2 * c.kv_dim()); }
 
 // Every layer for N tokens whose embeddings are in b.x (row stride hidden).
-// attend(l, w) computes layer l's attention from the raw projections b.q,
-// b.k, b.v into b.attn (and writes the cache). On return b.x holds the final
+// attend(l, w, pend) computes layer l's attention from the raw projections b.q,
+// b.k, b.v into b.attn (and writes the cache); where pend[i].part is set,
+// projection i is still in pending partial sums instead of its buffer. On return b.x holds the final
 // residual stream, every pending split-K sum applied.
 template <typename Attend>
 void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend) {
@@ -93,7 +94,9 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
     return k::DecodeMatvecBatch(a, stream);
   };
   auto project = [&](const float* in, int K, const float* norm_w,
-                     std::initializer_list<std::pair<const k::MatRef*, k::GemmJob>> jobs) {
+                     std::initializer_list<std::pair<const k::MatRef*, k::GemmJob>> jobs,
+                     k::SplitPending* out = nullptr) {
+    // (out: one entry per job, left pending where the launch splits K)
     bool all_gemm = mma;
     for (const auto& jb : jobs) all_gemm = all_gemm && k::QGemmSupports(*jb.first);
     if (in != x || !all_gemm) settle();
@@ -103,9 +106,11 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
       norm_w = nullptr;
     }
     k::GemmJob g[3];
-    int ng = 0;
+    int ng = 0, at[3] = {0, 0, 0}, ij = 0;  // at: job of g[i]
     for (const auto& jb : jobs) {
+      const int job = ij++;
       if (mma && k::QGemmSupports(*jb.first)) {
+        at[ng] = job;
         g[ng++] = jb.second;
       } else {
         k::Matvec(*jb.first, in, K, N, jb.second.y, jb.second.ldy, jb.second.epi, stream);
@@ -118,18 +123,21 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
     // one launch per weight type; a second type runs on the side stream
     // beside the first, each with half of the split-K partial buffer
     k::GemmJob grp[3][3];
-    int gn[3] = {0, 0, 0}, n_grp = 0;
+    int gn[3] = {0, 0, 0}, n_grp = 0, ga[3][3];
     bool done[3] = {false, false, false};
     for (int i = 0; i < ng; ++i) {
       if (done[i]) continue;
       for (int j = i; j < ng; ++j) {
         if (!done[j] && g[j].w.type == g[i].w.type) {
+          ga[n_grp][gn[n_grp]] = at[j];
           grp[n_grp][gn[n_grp]++] = g[j];
           done[j] = true;
         }
       }
       ++n_grp;
     }
+    k::SplitPending left[3][3];
+    k::SplitPending* const defer[3] = {out ? left[0] : nullptr, out ? left[1] : nullptr, nullptr};
     if (n_grp == 2) {
       k::SplitX sa = sx, sb = sx;
       sa.part_floats = sx.part_floats / 2;
@@ -142,15 +150,18 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
       for (int i = 0; i < 2; ++i)
         for (int j = 0; j < gn[i]; ++j) rows[i] += grp[i][j].w.rows;
       const int side_cus = std::max<int>(1, static_cast<int>(k::ComputeUnits() * rows[1] / (rows[0] + rows[1])));
-      k::QGemm(sb, grp[1], gn[1], b.side, nullptr, side_cus);
+      k::QGemm(sb, grp[1], gn[1], b.side, defer[1], side_cus);
       HIP_CHECK(hipEventRecord(b.ev_join, b.side));
-      k::QGemm(sa, grp[0], gn[0], stream, nullptr, std::max(1, k::ComputeUnits() - side_cus));
+      k::QGemm(sa, grp[0], gn[0], stream, defer[0], std::max(1, k::ComputeUnits() - side_cus));
       HIP_CHECK(hipStreamWaitEvent(stream, b.ev_join, 0));
     } else if (n_grp == 1 && gn[0] == 1 && grp[0][0].y == x && grp[0][0].epi == k::kAdd) {
       k::QGemm(sx, grp[0], 1, stream, &pend);  // a K split's sums stay pending
     } else {
-      for (int i = 0; i < n_grp; ++i) k::QGemm(sx, grp[i], gn[i], stream);
+      // (three types in turn share the partials' buffer: each is summed before the next)
+      for (int i = 0; i < n_grp; ++i) k::QGemm(sx, grp[i], gn[i], stream, n_grp == 1 ? defer[0] : nullptr);
     }
+    for (int i = 0; out != nullptr && i < std::min(n_grp, 2); ++i)
+      for (int j = 0; j < gn[i]; ++j) out[ga[i][j]] = left[i][j];
   };
   auto gj = [](const k::MatRef& w, float* y, int64_t ldy, k::Epilogue epi) {
     k::GemmJob j;
@@ -162,11 +173,12 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
   };
   for (int l = 0; l < c.n_layers; ++l) {
     const LayerDev& w = m.layers()[static_cast<size_t>(l)];
+    k::SplitPending qkv[3];
     if (!batch(x, H, w.attn_norm, false,
                {gj(w.dq, b.q, qd, k::kStore), gj(w.dk, b.k, kvd, k::kStore), gj(w.dv, b.v, kvd, k::kStore)}))
       project(x, H, w.attn_norm,
-              {gj(w.q, b.q, qd, k::kStore), gj(w.k, b.k, kvd, k::kStore), gj(w.v, b.v, kvd, k::kStore)});
-    attend(l, w);
+              {gj(w.q, b.q, qd, k::kStore), gj(w.k, b.k, kvd, k::kStore), gj(w.v, b.v, kvd, k::kStore)}, qkv);
+    attend(l, w, qkv);
     if (!batch(b.attn, qd, nullptr, false, {gj(w.dout, x, H, k::kAdd)}))
       project(b.attn, qd, nullptr, {gj(w.o, x, H, k::kAdd)});
     if (batch(x, H, w.ffn_norm, true, {gj(w.gate_up, b.act, F, k::kStore)})) {

@@ -56,9 +56,8 @@ typedef float F16v __attribute__((ext_vector_type(16)));
 typedef uint32_t U2 __attribute__((ext_vector_type(2)));
 typedef uint32_t U4 __attribute__((ext_vector_type(4)));
 
-constexpr int kThreads = 512;      // 8 waves: 2 token halves of 64 x 4 row quarters of 64
-constexpr int kTM = kTiledTokens;  // tokens per workgroup
-constexpr int kTN = kTiledRows;    // weight rows per workgroup
+constexpr int kThreads = 512;    // 8 waves
+constexpr int kTN = kTiledRows;  // weight rows per workgroup
 
 // 16 bytes at an address that is only 2-byte aligned (Q6_K and Q8_0 blocks
 // are 210 and 34 bytes long): one dwordx4 load, which global memory serves at
@@ -73,6 +72,11 @@ __device__ __forceinline__ T GLoad(const void* p) {
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 __device__ __forceinline__ Rsrc MakeRsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
+}
+
+// 16 bytes per lane from the resource to LDS (a wave's lanes side by side).
+__device__ __forceinline__ void DmaLds(Rsrc src, void* lds, uint32_t voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
 }
 
 // Chunk swizzle of the token rows in LDS (128-byte rows, 16-byte chunks):
@@ -102,6 +106,9 @@ __device__ __forceinline__ F16v MmaFresh(H8 a, H8 b) {
   asm volatile("" ::"v"(a), "v"(b), "v"(r));
   return r;
 }
+// Keeps the computation of t at its place.
+__device__ __forceinline__ void Pin(F16v& t) { asm volatile("" : "+v"(t)); }
+
 // (a & mask) | c with the mask in an SGPR (gfx9 VOP3 takes no literal).
 __device__ __forceinline__ uint32_t AndOr(uint32_t a, uint32_t mask, uint32_t c) {
   uint32_t r;
@@ -149,9 +156,16 @@ __device__ __forceinline__ H8 UnpackBytes(uint32_t v0, uint32_t v1, uint32_t mag
 // 128 h + 32 m + [0, 32) and 128 h + 64 + 32 m + [0, 32): low and high
 // nibbles of the same 32 ql bytes, with their qh bits); the token rows are
 // staged in that order. For Q8_0, two 32-weight blocks.
-template <int QT>
+//
+// kTM: tokens per workgroup. 128: waves in 2 token halves x 4 row quarters,
+// each 64 tokens x 64 rows; 64 (segments of up to 64 tokens, half the
+// products of a 128-token tile): 8 row eighths, each 64 tokens x 32 rows.
+template <int QT, int kTM>
 __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   constexpr bool kQ4 = QT == kQ4_K, kQ6 = QT == kQ6_K;
+  constexpr int kNI = kTM / 64;    // 32-row tiles per wave
+  constexpr int kWN = 32 * kNI;    // rows per wave
+  constexpr int kDma = kTM / 32;   // DMA loads of a step's token rows per wave
   // the tiles from tail_wg on in K parts: workgroup tail_wg + ts i + z takes
   // part z of tile tail_wg + i
   int wgi = static_cast<int>(blockIdx.x), zt = -1;
@@ -178,7 +192,7 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   const int m0 = tm * kTM;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 2, wn = wave & 3;  // 64-token half, 64-row quarter
+  const int wm = kNI == 2 ? wave >> 2 : 0, wn = kNI == 2 ? wave & 3 : wave;  // 64-token half, kWN rows
   const int l32 = lane & 31, lh = lane >> 5;
   const int rows = J.w.rows;
   const int64_t rb = J.w.row_bytes;
@@ -211,15 +225,17 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
 
   __shared__ __align__(16) float Is[kTM];  // 1 / s of the token rows
 
-  // The weight row this thread stages: local row br, half bq of a step
-  // (Q4_K: 16 of its 32 quant bytes; Q6_K: ql / qh bytes 16 bq .. + 16, slices
-  // bq and 2 + bq; Q8_0: block bq, slices 2 bq and 2 bq + 1). A pair's
-  // workgroup holds 128 output rows: local rows 64 h + [0, 32) are gate rows
-  // 128 nt + 32 h + [0, 32), 64 h + [32, 64) the same rows of up (so the
-  // matrix is wave-uniform: wave bit 0).
-  const int br = tid >> 1, bq = tid & 1;
+  // The weight row this thread stages, as local row br, and the half bq of a
+  // step (Q4_K: 16 of its 32 quant bytes; Q6_K: ql / qh bytes 16 bq .. + 16,
+  // slices bq and 2 + bq; Q8_0: block bq, slices 2 bq and 2 bq + 1). A pair's
+  // workgroup holds 128 output rows; even waves stage gate rows, odd ones up
+  // rows (the matrix is wave-uniform). A wave's rows are gate rows and then
+  // the same up rows: 32 + 32 as its two tiles, or 16 + 16 of its one.
+  const int bq = tid & 1, bi = (tid >> 1) & 31;
+  const int pr = 32 * (wave >> 1) + bi;  // (pair: row of the 128)
+  const int br = kNI == 1 && pair ? 32 * (pr >> 4) + 16 * (wave & 1) + (pr & 15) : tid >> 1;
   const uint8_t* bmat = (pair && (wave & 1)) ? a.job[1].w.w : J.w.w;
-  const int brow_i = pair ? min(128 * nt + 32 * (br >> 6) + (br & 31), rows - 1) : min(kTN * nt + br, rows - 1);
+  const int brow_i = pair ? min(128 * nt + pr, rows - 1) : min(kTN * nt + br, rows - 1);
   const Rsrc rwt = MakeRsrc(bmat, static_cast<uint32_t>(rows) * static_cast<uint32_t>(rb));
   const uint32_t b_off = static_cast<uint32_t>(brow_i) * static_cast<uint32_t>(rb);
   // (Q6_K, Q8_0: 2-byte aligned global loads, a uniform base and a 32-bit
@@ -227,25 +243,25 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   const uint32_t b_lane = b_off + (kQ6 ? 16u : 34u) * bq;
   // The token rows of a step reach LDS by DMA (buffer loads with an LDS
   // destination: a wave's 64 lanes x 16 bytes land as 1 KB in a row). A
-  // step's rows are 2 parts x 128 tokens x 128 bytes = 32 such loads, 4 per
-  // wave: load i of wave w fills part w / 4, rows 8 b .. 8 b + 7, b =
-  // (4 w + i) % 16; lane L reads token row 8 b + L / 8 and lands at chunk
+  // step's rows are 2 parts x kTM tokens x 128 bytes = kTM / 4 such loads,
+  // kDma per wave: load i of wave w fills part w / 4, rows 8 b .. 8 b + 7, b =
+  // (kDma w + i) % (kTM / 8); lane L reads token row 8 b + L / 8 and lands at chunk
   // L % 8 of it, which holds logical chunk (L % 8) ^ ASwz(row). Logical chunk
   // c holds step inputs 8 c .. + 8 (Q6_K: 8 c and 32 + 8 c of the step's two
   // strips). The buffer resources end at the last token, so the rows past it
   // read as zeros.
   const uint32_t a_bytes = static_cast<uint32_t>(M) * static_cast<uint32_t>(K) * 2u;
   const Rsrc ra_src = MakeRsrc(wave < 4 ? x.hi : x.lo, a_bytes);
-  uint32_t a_voff[4];
+  uint32_t a_voff[kDma];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = 8 * ((4 * wave + i) & 15) + (lane >> 3);
+  for (int i = 0; i < kDma; ++i) {
+    const int r = 8 * ((kDma * wave + i) & (kTM / 8 - 1)) + (lane >> 3);
     const int lc = (lane & 7) ^ ASwz(r);
     a_voff[i] = (static_cast<uint32_t>(m0 + r) * static_cast<uint32_t>(K) + 8u * lc + (kQ6 && lc >= 4 ? 32u : 0u)) * 2u;
   }
-  // Q4_K sub-block sums: part x token, one chunk of 8 (threads 256.. repeat
-  // 0..255)
-  const int sp = (wave >> 1) & 1, sr = tid & (kTM - 1);
+  // Q4_K sub-block sums: part x token, one chunk of 8 (threads 2 kTM ..
+  // repeat the first)
+  const int sp = (wave / kNI) & 1, sr = tid & (kTM - 1);
   const Rsrc rsum = MakeRsrc(sp ? x.sum_lo : x.sum_hi, static_cast<uint32_t>(M) * static_cast<uint32_t>(K >> 5) * 2u);
   const uint32_t s_off = static_cast<uint32_t>(m0 + sr) * static_cast<uint32_t>(K >> 5) * 2u;
 
@@ -274,16 +290,14 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   // longer, more would let a step read rows still in flight)
   constexpr int kLoads0 = kQ4 ? 3 : kQ6 ? 4 : 3, kLoads1 = kQ4 ? 1 : kQ6 ? 2 : 3;
   // the token rows of step g (g = 4 o + s of this part, super-block o0 + o)
-  // into stage st (4 DMA loads per wave)
+  // into stage st
   auto issue_a = [&](int g, int st) {
     g = min(g, nsteps - 1);
     const int ob = o0 + (g >> 2), s = g & 3;
     const int so = kQ6 ? 2 * (256 * ob + 128 * (s >> 1) + 32 * (s & 1)) : 2 * (256 * ob + 64 * s);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          ra_src, (__attribute__((address_space(3))) void*)(&as(st)[wave >> 2][8 * ((4 * wave + i) & 15)][0]),
-          16, a_voff[i], so, 0, 0);
+    for (int i = 0; i < kDma; ++i)
+      DmaLds(ra_src, &as(st)[wave >> 2][8 * ((kDma * wave + i) & (kTM / 8 - 1))][0], a_voff[i], so);
   };
   // (ss = g % 4, known at compile time at every call)
   auto issue = [&](int g, int slot, int ss) {
@@ -390,22 +404,22 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   // weights and is subtracted: the two halves' errors cancel. The min terms
   // alternate by super-block.
   constexpr int kGl = kQ6 ? 0 : 1, kGroup = 1 << kGl;
-  F16v T[2][2], P[2][2];
-  float Cs[2] = {0.0f, 0.0f};
+  F16v T[2][kNI], P[2][kNI];
+  float Cs[kNI] = {};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    T[i >> 1][i & 1] = F16v{};
-    P[i >> 1][i & 1] = F16v{};
+  for (int i = 0; i < 2 * kNI; ++i) {
+    T[i / kNI][i % kNI] = F16v{};
+    P[i / kNI][i % kNI] = F16v{};
   }
 
   // token operands of one slice and part, double-buffered; the weight
   // operands of a group
-  H8 op[2][2], b[kGroup][2];
-  // quants of the wave's 64 rows (and Q4_K scale pairs, Q6_K / Q8_0 scales):
+  H8 op[2][2], b[kGroup][kNI];
+  // quants of the wave's rows (and Q4_K scale pairs, Q6_K / Q8_0 scales):
   // Q4_K a whole step; else slices 2 p and 2 p + 1
-  U4 qv[2];
-  U2 s4[2];
-  float sc[2][2];
+  U4 qv[kNI];
+  U2 s4[kNI];
+  float sc[kNI][2];
   // Q4_K's lane half lh takes quant bytes 16 lh .. + 16: slice kk multiplies
   // logical token chunk 4 (kk / 2) + 2 lh + kk % 2, else 2 kk + lh
   auto read_a = [&](H8* q, int st, int part, int kk) {
@@ -418,8 +432,8 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   };
   auto read_q = [&](int st, int p, int tb, int s) {
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-      const int r = 64 * wn + 32 * ni + l32;
+    for (int ni = 0; ni < kNI; ++ni) {
+      const int r = kWN * wn + 32 * ni + l32;
       qv[ni] = Bq[st][kQ4 ? lh : 2 * p + lh][r];
       if constexpr (kQ4) {
         s4[ni] = S4[tb][s][r];
@@ -450,7 +464,7 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   read_q(0, 0, 0, 0);
   if constexpr (kQ4) {
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni) sc[ni][0] = Dd[0][64 * wn + 32 * ni + l32].x;
+    for (int ni = 0; ni < kNI; ++ni) sc[ni][0] = Dd[0][kWN * wn + 32 * ni + l32].x;
   }
   for (int o = 0; o < o1 - o0; ++o) {
     const int tb = o & 1;
@@ -464,8 +478,8 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
       // step g + 2's DMA is issued.
       const int g = 4 * o + s, st = s & 1, nx = st ^ 1, ns = (s + 1) & 3;
       // Q4_K, the super-block's end: its mins, -32 dmin and sub-block sums
-      H8 bm[2], xs[2];
-      float dm[2];
+      H8 bm[kNI], xs[2];
+      float dm[kNI];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int kk = ((i >> (kGl + 1)) << kGl) | (i & (kGroup - 1)), hi = (i >> kGl) & 1;
@@ -480,13 +494,15 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
           __syncthreads();
           if (kQ4 && s == 3) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-              const int r = 64 * wn + 32 * t + l32;
+            for (int t = 0; t < kNI; ++t) {
+              const int r = kWN * wn + 32 * t + l32;
               bm[t] = *reinterpret_cast<const H8*>(&Mn[tb][r][0]);
               dm[t] = Dd[tb][r].y;  // (its sign the mins')
               sc[t][0] = Dd[tb ^ 1][r].x;
-              xs[t] = *reinterpret_cast<const H8*>(&Ss[tb][lh][64 * wm + 32 * t + l32][0]);
             }
+#pragma unroll
+            for (int mi = 0; mi < 2; ++mi)
+              xs[mi] = *reinterpret_cast<const H8*>(&Ss[tb][lh][64 * wm + 32 * mi + l32][0]);
           }
           read_a(op[0], nx, 1, 0);
         } else {
@@ -495,7 +511,7 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
         }
         if (!hi) {
 #pragma unroll
-          for (int ni = 0; ni < 2; ++ni) {
+          for (int ni = 0; ni < kNI; ++ni) {
             const uint32_t v0 = qv[ni][2 * (kk & 1)], v1 = qv[ni][2 * (kk & 1) + 1];
             if constexpr (kQ4)
               b[kg][ni] = UnpackQ4(v0, v1, kk < 2 ? mlo : mhi, magic, kk < 2 ? s4[ni].x : s4[ni].y);
@@ -509,13 +525,13 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
 #pragma unroll
         for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-          for (int ni = 0; ni < 2; ++ni) {
+          for (int ni = 0; ni < kNI; ++ni) {
             if (fresh) {
 #pragma unroll
               for (int v = 0; v < 16; ++v)
                 T[mi][ni][v] = __builtin_fmaf(last_neg ? -Cs[ni] : Cs[ni], P[mi][ni][v], T[mi][ni][v]);
               // (here, not later: the compiler would else keep both P)
-              asm volatile("" : "+v"(T[mi][ni]));
+              Pin(T[mi][ni]);
               P[mi][ni] = MmaFresh(q[mi], b[kg][ni]);
               __builtin_amdgcn_sched_barrier(0);  // (a tile's sums scaled, then overwritten)
             } else {
@@ -523,8 +539,8 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
             }
           }
         if (fresh) {
-          Cs[0] = sc[0][kQ6 ? kk & 1 : 0];
-          Cs[1] = sc[1][kQ6 ? kk & 1 : 0];
+#pragma unroll
+          for (int ni = 0; ni < kNI; ++ni) Cs[ni] = sc[ni][kQ6 ? kk & 1 : 0];
         }
         // the next step's staging, spread over the items
         if (i == 1 && s == 3) store_tables(tb ^ 1);  // step g + 1 starts super-block o + 1
@@ -546,7 +562,7 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
 #pragma unroll
         for (int mi = 0; mi < 2; ++mi) {
 #pragma unroll
-          for (int ni = 0; ni < 2; ++ni) {
+          for (int ni = 0; ni < kNI; ++ni) {
             const F16v qm = MmaFresh(xs[mi], bm[ni]);
 #pragma unroll
             for (int v = 0; v < 16; ++v) T[mi][ni][v] = __builtin_fmaf(dm[ni], qm[v], T[mi][ni][v]);
@@ -557,11 +573,12 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   }
 
   // epilogue: result v of tile (mi, ni) is token 64 wm + 32 mi + 8 (v / 4) +
-  // 4 lh + v % 4, local row 64 wn + 32 ni + l32
+  // 4 lh + v % 4, local row kWN wn + 32 ni + l32
+  constexpr int kHalf = kWN / 2;  // a pair: gate rows of the wave, then its up rows
 #pragma unroll
   for (int mi = 0; mi < 2; ++mi) {
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
+    for (int ni = 0; ni < kNI; ++ni)
 #pragma unroll
       for (int v = 0; v < 16; ++v) T[mi][ni][v] = __builtin_fmaf(-Cs[ni], P[mi][ni][v], T[mi][ni][v]);  // (an odd one)
     // a quad of tokens at a time: 8 (v / 4) + 4 lh + [0, 4)
@@ -572,29 +589,33 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
       const float is[4] = {is4.x, is4.y, is4.z, is4.w};
       if (zt >= 0) {
         // a part of a tail tile: raw sums, [token][local row]
-        float* pt = x.part + (static_cast<int64_t>(wgi - a.tail_wg) * ts + zt) * kTiledTailFloats + t0 * kTN +
-                    64 * wn + l32;
+        float* pt = x.part + (static_cast<int64_t>(wgi - a.tail_wg) * ts + zt) * (kTM * kTN) + t0 * kTN + kWN * wn + l32;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          pt[e * kTN] = T[mi][0][4 * v4 + e];
-          pt[e * kTN + 32] = T[mi][1][4 * v4 + e];
-        }
+        for (int ni = 0; ni < kNI; ++ni)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) pt[e * kTN + 32 * ni] = T[mi][ni][4 * v4 + e];
       } else if (pair) {
-        // gate (tile 0) and up (tile 1) of the same row: silu(g) * u
-        // (reference src/kernels.h:82-92), the bits of the unfused stores
-        // followed by SwiGLURows
-        const int row = 128 * nt + 32 * wn + l32;
+        // gate and up of the same row -- tiles 0 and 1, or lanes l32 and l32 +
+        // 16 of the one tile: silu(g) * u (reference src/kernels.h:82-92), the
+        // bits of the unfused stores followed by SwiGLURows
+        const int row = 128 * nt + kHalf * wn + l32 % kHalf;
         float* y = J.y + static_cast<int64_t>(m0 + t0) * J.ldy + row;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float g = T[mi][0][4 * v4 + e] * is[e], u = T[mi][1][4 * v4 + e] * is[e];
+          const float tg = T[mi][0][4 * v4 + e];
+          float tu;
+          if constexpr (kNI == 2)
+            tu = T[mi][kNI - 1][4 * v4 + e];
+          else
+            tu = __shfl_xor(tg, 16, 64);
+          const float g = tg * is[e], u = tu * is[e];
           const float sg = g / __fadd_rn(1.0f, GlibcExpf(-g));
-          if (row < rows && m0 + t0 + e < M) y[e * J.ldy] = __fmul_rn(sg, u);
+          if (row < rows && m0 + t0 + e < M && l32 < kHalf) y[e * J.ldy] = __fmul_rn(sg, u);
         }
       } else {
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
-          const int row = kTN * nt + 64 * wn + 32 * ni + l32;
+        for (int ni = 0; ni < kNI; ++ni) {
+          const int row = kTN * nt + kWN * wn + 32 * ni + l32;
           float val[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) val[e] = T[mi][ni][4 * v4 + e] * is[e];
@@ -627,22 +648,24 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
 // tile's K parts (added in part order, then scaled as the full tiles' sums
 // are), the full tiles' SwiGLU arithmetic. Workgroup (tile, y) takes tokens
 // 8 y .. 8 y + 7 of the tile, four outputs per thread.
-constexpr int kTailPer = 4, kTailSlices = kTM * (kTN / 2) / (256 * kTailPer);
+constexpr int kTailPer = 4;
+template <int kTM>
 __global__ __launch_bounds__(256) void TailSwiGLUKernel(TiledArgs a) {
+  constexpr int kHalf = 16 * (kTM / 64);  // a wave's gate rows, followed by its up rows
   const int tt = static_cast<int>(blockIdx.x), tile = a.tail_wg + tt;
   const int tm = tile % a.tiles_m, nt = tile / a.tiles_m;
   const GemmJob& J = a.job[0];
   const int rows = J.w.rows, M = a.x.M;
-  const float* p = a.x.part + static_cast<int64_t>(tt) * a.tail_split * kTiledTailFloats;
+  const float* p = a.x.part + static_cast<int64_t>(tt) * a.tail_split * (kTM * kTN);
   float g[kTailPer], u[kTailPer], is[kTailPer];
 #pragma unroll
   for (int i = 0; i < kTailPer; ++i) {
     const int e = (static_cast<int>(blockIdx.y) * kTailPer + i) * 256 + static_cast<int>(threadIdx.x);
     const int tl = e >> 7, c = e & 127;
     // (tokens past M were not stored: their sums are read but not used)
-    const float* q = p + tl * kTN + 64 * (c >> 5) + (c & 31);
+    const float* q = p + tl * kTN + 2 * kHalf * (c / kHalf) + c % kHalf;
     g[i] = q[0];
-    u[i] = q[32];
+    u[i] = q[kHalf];
     is[i] = a.x.inv_s[min(tm * kTM + tl, M - 1)];
   }
   for (int z = 1; z < a.tail_split; ++z) {
@@ -650,9 +673,9 @@ __global__ __launch_bounds__(256) void TailSwiGLUKernel(TiledArgs a) {
     for (int i = 0; i < kTailPer; ++i) {
       const int e = (static_cast<int>(blockIdx.y) * kTailPer + i) * 256 + static_cast<int>(threadIdx.x);
       const int tl = e >> 7, c = e & 127;
-      const float* q = p + static_cast<int64_t>(z) * kTiledTailFloats + tl * kTN + 64 * (c >> 5) + (c & 31);
+      const float* q = p + static_cast<int64_t>(z) * (kTM * kTN) + tl * kTN + 2 * kHalf * (c / kHalf) + c % kHalf;
       g[i] += q[0];
-      u[i] += q[32];
+      u[i] += q[kHalf];
     }
   }
 #pragma unroll
@@ -677,22 +700,40 @@ void LaunchTiled(const TiledArgs& a, hipStream_t s) {
   for (int j = 1; j < a.n_jobs + (a.pair ? 1 : 0); ++j)
     RPG_CHECK(a.job[j].w.type == type, "tiled gemm: one weight type per launch");
   RPG_CHECK(a.x.K % 256 == 0 && a.x.K >= 256, "tiled gemm: K = %d is not a multiple of 256", a.x.K);
+  RPG_CHECK(a.tokens == TiledTokens(a.x.M) && a.tiles_m == CeilDiv(a.x.M, a.tokens), "tiled gemm: bad token tiles");
   RPG_CHECK(a.ksplit >= 1 && a.ksplit <= a.x.K / 256, "tiled gemm: bad K split %d", a.ksplit);
   const int total = tiles * a.tiles_m;
   const int n_tail = a.tail_split > 1 ? total - a.tail_wg : 0;
   if (a.tail_split > 1)
     RPG_CHECK(a.pair && a.ksplit == 1 && a.tail_wg >= 0 && a.tail_wg < total && a.tail_split <= a.x.K / 256 &&
-                  static_cast<int64_t>(n_tail) * a.tail_split * kTiledTailFloats <= a.x.part_floats,
+                  static_cast<int64_t>(n_tail) * a.tail_split * a.tokens * kTN <= a.x.part_floats,
               "tiled gemm: bad tail split %d from workgroup %d of %d", a.tail_split, a.tail_wg, total);
   const dim3 grid(static_cast<unsigned>(total + n_tail * (a.tail_split - 1)), static_cast<unsigned>(a.ksplit));
-  switch (type) {
-    case kQ4_K: hipLaunchKernelGGL(TGemmKernel<kQ4_K>, grid, dim3(kThreads), 0, s, a); break;
-    case kQ6_K: hipLaunchKernelGGL(TGemmKernel<kQ6_K>, grid, dim3(kThreads), 0, s, a); break;
-    default: hipLaunchKernelGGL(TGemmKernel<kQ8_0>, grid, dim3(kThreads), 0, s, a);
+  const bool small = a.tokens == 64;
+  const dim3 block(kThreads);
+  if (type == kQ4_K) {
+    if (small)
+      hipLaunchKernelGGL((TGemmKernel<kQ4_K, 64>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((TGemmKernel<kQ4_K, 128>), grid, block, 0, s, a);
+  } else if (type == kQ6_K) {
+    if (small)
+      hipLaunchKernelGGL((TGemmKernel<kQ6_K, 64>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((TGemmKernel<kQ6_K, 128>), grid, block, 0, s, a);
+  } else {
+    if (small)
+      hipLaunchKernelGGL((TGemmKernel<kQ8_0, 64>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((TGemmKernel<kQ8_0, 128>), grid, block, 0, s, a);
   }
   HIP_CHECK(hipGetLastError());
   if (n_tail > 0) {
-    hipLaunchKernelGGL(TailSwiGLUKernel, dim3(static_cast<unsigned>(n_tail), kTailSlices), dim3(256), 0, s, a);
+    const dim3 tail_grid(static_cast<unsigned>(n_tail), static_cast<unsigned>(a.tokens * (kTN / 2) / (256 * kTailPer)));
+    if (small)
+      hipLaunchKernelGGL(TailSwiGLUKernel<64>, tail_grid, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL(TailSwiGLUKernel<128>, tail_grid, dim3(256), 0, s, a);
     HIP_CHECK(hipGetLastError());
   }
 }

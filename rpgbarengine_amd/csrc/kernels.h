@@ -62,6 +62,15 @@ void Dequant(uint32_t type, const uint8_t* src, int64_t n, float* dst, hipStream
 void RmsNormRows(const float* x, int64_t ldx, const float* w, int n, int rows, float eps, float* out,
                  int64_t ldo, hipStream_t s);
 
+// Split-K partial sums of a projection not yet in its output: output column c
+// of token t is the sum over z < ksplit of part[(z * M + t) * part_ld + pcol + c].
+constexpr int kMaxPendParts = 8;
+struct SplitPending {
+  const float* part = nullptr;
+  int64_t part_ld = 0;
+  int32_t pcol = 0, ksplit = 1, M = 0;
+};
+
 // Per token t of a segment starting at absolute position pos0 (device scalar
 // when pos0_dev != nullptr, else pos0_host): RMSNorm every Q and K head with
 // q_norm / k_norm, RoPE with the table row of position pos0+t, write K and V
@@ -80,6 +89,9 @@ struct QkvArgs {
   float eps;
   const int32_t* pos0_dev;
   int32_t pos0_host;
+  // q, k, v still as pending partial sums (part != null): summed here, in
+  // split order, instead of read from the buffers above
+  SplitPending pend[3];
 };
 void QkNormRopeCache(const QkvArgs& a, hipStream_t s);
 

@@ -358,6 +358,24 @@ __global__ __launch_bounds__(256) void RmsNormKernel(const float* __restrict__ x
 
 // ---------------------------------------------------------------- QK-norm + RoPE + cache
 
+// Columns col and col + 64 of token t of a projection: from its pending
+// partial sums (every one requested before the first is added), else from
+// src.
+__device__ __forceinline__ float2 PendPair(const SplitPending& p, int t, int col, const float* src) {
+  if (p.part == nullptr) return float2{src[0], src[64]};
+  const float* q = p.part + static_cast<int64_t>(t) * p.part_ld + p.pcol + col;
+  const int64_t step = static_cast<int64_t>(p.M) * p.part_ld;
+  float a[kMaxPendParts], b[kMaxPendParts];
+#pragma unroll
+  for (int z = 0; z < kMaxPendParts; ++z)
+    if (z < p.ksplit) a[z] = q[z * step], b[z] = q[z * step + 64];
+  float2 v = {0.0f, 0.0f};
+#pragma unroll
+  for (int z = 0; z < kMaxPendParts; ++z)
+    if (z < p.ksplit) v.x += a[z], v.y += b[z];
+  return v;
+}
+
 // grid (n_heads + n_kv, seq), 64 threads: lane i holds the RoPE pair (i, i + hd/2)
 // for hd = 128.
 __global__ __launch_bounds__(64) void QkNormRopeKernel(QkvArgs a) {
@@ -371,7 +389,8 @@ __global__ __launch_bounds__(64) void QkNormRopeKernel(QkvArgs a) {
   const float* src = is_q ? a.q + (static_cast<int64_t>(t) * a.n_heads + head) * a.hd
                           : a.k + (static_cast<int64_t>(t) * a.n_kv + head) * a.hd;
   const float* nw = is_q ? a.q_norm : a.k_norm;
-  const float x0 = src[i], x1 = src[i + half];
+  const float2 x = PendPair(a.pend[is_q ? 0 : 1], t, head * a.hd + i, src + i);
+  const float x0 = x.x, x1 = x.y;
   double s = static_cast<double>(x0) * x0 + static_cast<double>(x1) * x1;
   s = WaveSumD(s);
   const double mean = s / static_cast<double>(a.hd);
@@ -393,8 +412,9 @@ __global__ __launch_bounds__(64) void QkNormRopeKernel(QkvArgs a) {
     const float* vs = a.v + (static_cast<int64_t>(t) * a.n_kv + head) * a.hd;
     kd[i] = ra;
     kd[i + half] = rb;
-    vd[i] = vs[i];
-    vd[i + half] = vs[i + half];
+    const float2 v = PendPair(a.pend[2], t, head * a.hd + i, vs + i);
+    vd[i] = v.x;
+    vd[i + half] = v.y;
   }
 }
 
@@ -653,6 +673,9 @@ void RmsNormRows(const float* x, int64_t ldx, const float* w, int n, int rows, f
 void QkNormRopeCache(const QkvArgs& a, hipStream_t s) {
   RPG_CHECK(a.hd == 128, "QK-norm/RoPE kernel is built for head_dim 128 (got %d)", a.hd);
   if (a.seq <= 0) return;
+  for (const SplitPending& p : a.pend)
+    RPG_CHECK(p.part == nullptr || (p.M == a.seq && p.ksplit >= 1 && p.ksplit <= kMaxPendParts),
+              "QK-norm/RoPE: pending sums do not match the segment");
   hipLaunchKernelGGL(QkNormRopeKernel, dim3(static_cast<unsigned>(a.n_heads + a.n_kv), static_cast<unsigned>(a.seq)),
                      dim3(64), 0, s, a);
   HIP_CHECK(hipGetLastError());

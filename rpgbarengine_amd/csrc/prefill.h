@@ -53,19 +53,13 @@ SplitX SplitXView(void* base, int M, int K, int n_max);
 void SplitRows(const float* X, int64_t ldx, int M, int K, const float* norm_w, float eps, const SplitX& out,
                hipStream_t s);
 
-// Split-K partial sums of a kAdd projection not yet added to its output:
-// y[t][c] += sum over z < ksplit of part[(z * M + t) * part_ld + pcol + c].
-struct SplitPending {
-  const float* part = nullptr;
-  int64_t part_ld = 0;
-  int32_t pcol = 0, ksplit = 1, M = 0;
-};
 // SplitRows over X after adding the pending sums to X (written back: X is
 // the residual stream), the bits of the reduce launch followed by SplitRows.
 void SplitRowsAdd(float* X, int64_t ldx, int M, int K, const float* norm_w, float eps, const SplitX& out,
                   const SplitPending& pend, hipStream_t s);
-// The reduce launch of a pending sum, into y (row stride ldy, N columns).
-void ApplyPending(const SplitPending& pend, float* y, int64_t ldy, int N, hipStream_t s);
+// The reduce launch of a pending sum, added to or stored in y (row stride ldy,
+// N columns).
+void ApplyPending(const SplitPending& pend, float* y, int64_t ldy, int N, hipStream_t s, Epilogue epi = kAdd);
 
 // Compute units of the current device (queried once per device).
 int ComputeUnits();
@@ -82,44 +76,46 @@ bool QGemmSupports(const MatRef& w);
 // runs beside it.
 void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, SplitPending* defer = nullptr,
            int cus = 0);
-// (defer: for one kAdd job, a K split's sums are left to the caller -- to
-// SplitRowsAdd or ApplyPending before y is read; defer->ksplit stays 1 when
-// nothing is pending)
+// (defer: one entry per job; a K split's sums are left to the caller, to add
+// or store before y is read -- SplitRowsAdd, QkNormRopeCache, ApplyPending.
+// defer[j].part stays null when nothing is pending)
 // gate.y[t][r] = silu(gate row r . x_t) * (up row r . x_t) in one launch,
 // the same bits as two QGemm products and SwiGLURows -- except where a tiled
 // launch runs its last round's tiles in K parts: those rows' sums are the
 // parts' sums added, within the products' row bound. Gate and up of one type
-// and shape; Q4_K, or any type of the tiled launch where that takes the
-// segment, and only where the 32-token kernel would not split K; false
-// (nothing launched) otherwise.
+// and shape that the tiled launch takes; false (nothing launched) otherwise.
 bool QGemmSwiGLU(const SplitX& x, const GemmJob& gate, const GemmJob& up, hipStream_t s);
 
 // y[i] = silu(g[i]) * u[i] (reference src/kernels.h:82-92), n elements.
 void SwiGLURows(const float* g, const float* u, float* y, int64_t n, hipStream_t s);
 
-// Tiled GEMM (gemm_tiled.hip; Q4_K, Q6_K, Q8_0): 128 tokens x 256 weight rows
-// per workgroup. QGemm and QGemmSwiGLU take it for segments of at least
-// kTiledMinTokens tokens.
-constexpr int kTiledTokens = 128;
+// Tiled GEMM (gemm_tiled.hip; Q4_K, Q6_K, Q8_0 with K a multiple of 256): 64 or
+// 128 tokens x 256 weight rows per workgroup. The K-quants' GEMM at every
+// segment length, and Q8_0's at those widths. Tiles of 64 tokens fill the
+// compute units with fewer K parts and pad less; from about 320 tokens on the
+// 128-token tiles' fewer LDS bytes per product win (a segment behind 600
+// tokens, ms, 64 / 128-token tiles: 4B Q4_K_M 65 tokens 7.4 / 8.7, 160 8.1 /
+// 10.2, 203 10.0 / 10.7, 300 11.8 / 12.0, 384 13.3 / 12.9, 512 16.2 / 15.5;
+// 1.7B Q4_K_M 65 4.7 / 5.9, 300 6.2 / 7.5, 512 8.7 / 8.8).
 constexpr int kTiledRows = 256;
-constexpr int kTiledMinTokens = 96;
+inline int TiledTokens(int M) { return M <= 320 ? 64 : 128; }
 
 struct TiledArgs {
   SplitX x;
   GemmJob job[3];
   int32_t tiles[3];  // 256-row tiles per job (pair: 128-row tiles of gate and up)
   int32_t n_jobs;
-  int32_t tiles_m;   // 128-token tiles; workgroup i takes token tile i % tiles_m
+  int32_t tokens;    // TiledTokens(x.M)
+  int32_t tiles_m;   // token tiles; workgroup i takes token tile i % tiles_m
   int32_t ksplit;    // blockIdx.y takes super-blocks [y * n / ksplit, (y + 1) * n / ksplit)
   int64_t part_ld;   // partials: x.part[(z * M + token) * part_ld + pcol[job] + row]
   int32_t pcol[3];
   int32_t pair;      // job 0 gate, job 1 up: y = silu(gate.x) * (up.x), no K split
   // pair only, tail_split > 1: the tiles from tail_wg on run as tail_split K
-  // parts each (raw sums to x.part, kTiledTailFloats per part), finished by
-  // a second launch
+  // parts each (raw sums to x.part, tokens x kTiledRows floats per part),
+  // finished by a second launch
   int32_t tail_wg = 0, tail_split = 1;
 };
-constexpr int kTiledTailFloats = kTiledTokens * kTiledRows;
 void LaunchTiled(const TiledArgs& a, hipStream_t s);
 
 }  // namespace k

@@ -22,10 +22,6 @@ constexpr int64_t kPrefillChunk = 4096;
 // Tokens per pass when every position's logits are returned (the logits
 // buffer holds a row per token of the pass, 0.6 MB each).
 constexpr int64_t kLogitRowsChunk = 512;
-// Least size of the operand buffer, whose room between projections holds the
-// partial states of a short segment's attention (37 tokens of the 4B shape
-// in 26 key ranges).
-constexpr size_t kAttnPartBytes = size_t{16} << 20;
 constexpr int kGenChunk = 16;           // decode steps between host stop checks
 // The persistent decode step needs every one of its workgroups resident at
 // once; two of them running together (sessions generating from different
@@ -267,8 +263,7 @@ void Session::EnsureScratch(int64_t tokens, int64_t logit_rows) {
   if (tokens >= 2) {  // GEMM operands of multi-token segments
     alloc(&gu_, 2 * static_cast<int64_t>(c.intermediate));
     const int kmax = std::max({c.hidden, c.q_dim(), c.intermediate});
-    const size_t split_bytes =
-        std::max(k::SplitXBytes(static_cast<int>(tokens), kmax, SplitColumns(c)), kAttnPartBytes);
+    const size_t split_bytes = k::SplitXBytes(static_cast<int>(tokens), kmax, SplitColumns(c));
     DeviceAlloc(&split_, split_bytes);
     split_bytes_ = static_cast<int64_t>(split_bytes);
   }
@@ -298,7 +293,7 @@ void Session::ForwardSegment(const int32_t* ids_dev, int64_t n, int64_t pos0, co
             (long long)logit_rows_cap_);
   k::GatherRows(m_.embd(), ids_dev, N, x_, H, d_err_, stream_);
   const FwdBufs b{x_, h_, q_, k_, v_, attn_, act_, gu_, split_, SplitColumns(c), stream_, side_, ev_fork_, ev_join_};
-  ForwardLayers(m_, b, N, [&](int l, const LayerDev& w) {
+  ForwardLayers(m_, b, N, [&](int l, const LayerDev& w, const k::SplitPending* pend) {
     k::QkvArgs qa;
     qa.q = q_;
     qa.k = k_;
@@ -316,6 +311,7 @@ void Session::ForwardSegment(const int32_t* ids_dev, int64_t n, int64_t pos0, co
     qa.eps = c.rms_eps;
     qa.pos0_dev = pos_dev;
     qa.pos0_host = static_cast<int32_t>(pos0);
+    for (int i = 0; i < 3; ++i) qa.pend[i] = pend[i];
     k::QkNormRopeCache(qa, stream_);
     k::AttnArgs aa;
     aa.q = q_;
