@@ -120,15 +120,16 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
     const k::SplitX sx = k::SplitXView(b.split, N, K, b.split_cols);
     k::SplitRowsAdd(const_cast<float*>(in), K, N, K, norm_w, c.rms_eps, sx, pend, stream);
     pend = k::SplitPending{};
-    // one launch per weight type; a second type runs on the side stream
-    // beside the first, each with half of the split-K partial buffer
+    // one launch per weight type (Q4_K and Q6_K share one); a second type runs
+    // on the side stream beside the first, each with half of the split-K
+    // partial buffer
     k::GemmJob grp[3][3];
     int gn[3] = {0, 0, 0}, n_grp = 0, ga[3][3];
     bool done[3] = {false, false, false};
     for (int i = 0; i < ng; ++i) {
       if (done[i]) continue;
       for (int j = i; j < ng; ++j) {
-        if (!done[j] && g[j].w.type == g[i].w.type) {
+        if (!done[j] && k::QGemmShares(g[j].w, g[i].w)) {
           ga[n_grp][gn[n_grp]] = at[j];
           grp[n_grp][gn[n_grp]++] = g[j];
           done[j] = true;

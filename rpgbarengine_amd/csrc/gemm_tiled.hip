@@ -161,27 +161,40 @@ __device__ __forceinline__ H8 UnpackBytes(uint32_t v0, uint32_t v1, uint32_t mag
 // each 64 tokens x 64 rows; 64 (segments of up to 64 tokens, half the
 // products of a 128-token tile): 8 row eighths, each 64 tokens x 32 rows.
 template <int QT, int kTM>
-__global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
+struct TileLds {
+  static constexpr bool kQ4 = QT == kQ4_K, kQ6 = QT == kQ6_K;
+  // quants of a step, 16-byte chunks side by side over the rows (a wave's
+  // reads of one chunk are 512 consecutive bytes):
+  //  Q4_K [stage][h][row]: bytes 16 h .. + 16 of the row's 32;
+  //  else [stage][2 p + h][row]: unsigned bytes, inputs 8 h .. + 8 of slices
+  //  2 p and 2 p + 1 (slice: 16 inputs of the step)
+  U4 Bq[2][kQ4 ? 2 : 4][kTN];
+  // Q4_K [table][step][row]: UnpackQ4's pairs of the step's two sub-blocks
+  U2 S4[kQ4 ? 2 : 1][4][kQ4 ? kTN : 1];
+  _Float16 Ss[kQ4 ? 2 : 1][2][kQ4 ? kTM : 1][8];  // Q4_K [table][hi, lo][token]: sub-block sums
+  _Float16 Mn[kQ4 ? 2 : 1][kQ4 ? kTN : 1][8];     // Q4_K [table][row]: integer mins
+  float2 Dd[kQ4 ? 2 : 1][kQ4 ? kTN : 1];          // Q4_K [table][row]: d, -32 dmin
+  // Q6_K [4 table + step][row]: d * sc of the step's 4 slices; Q8_0
+  // [stage][row]: d of its 2 blocks
+  static constexpr int kSc = kQ4 ? 1 : kQ6 ? 4 : 2;
+  alignas(16) float Sc[kQ4 ? 1 : kQ6 ? 8 : 2][kQ4 ? 1 : kTN][kSc];
+  alignas(16) float Is[kTM];  // 1 / s of the token rows
+};
+
+// Part zt of the tile's K (zt < 0: this launch's part blockIdx.y), tile (tm,
+// nt) of job j. As0, As1: a stage's token rows [hi, lo][token] each, swizzled
+// (ASwz): one array per stage, since the compiler tells LDS arrays apart when
+// it places the waits for its DMA loads, so that reads of one stage do not
+// wait for the DMA into the other.
+template <int QT, int kTM>
+__device__ __forceinline__ void TGemmTile(const TiledArgs& a, int wgi, int zt, int tm, int nt, int j,
+                                          _Float16 (&As0)[2][kTM][64], _Float16 (&As1)[2][kTM][64],
+                                          TileLds<QT, kTM>& L) {
   constexpr bool kQ4 = QT == kQ4_K, kQ6 = QT == kQ6_K;
   constexpr int kNI = kTM / 64;    // 32-row tiles per wave
   constexpr int kWN = 32 * kNI;    // rows per wave
   constexpr int kDma = kTM / 32;   // DMA loads of a step's token rows per wave
-  // the tiles from tail_wg on in K parts: workgroup tail_wg + ts i + z takes
-  // part z of tile tail_wg + i
-  int wgi = static_cast<int>(blockIdx.x), zt = -1;
   const int ts = a.tail_split;
-  if (ts > 1 && wgi >= a.tail_wg) {
-    const int u = wgi - a.tail_wg;
-    wgi = u / ts;
-    zt = u - wgi * ts;
-    wgi += a.tail_wg;
-  }
-  const int tm = wgi % a.tiles_m;
-  int nt = wgi / a.tiles_m, j = 0;
-  while (j + 1 < a.n_jobs && nt >= a.tiles[j]) {
-    nt -= a.tiles[j];
-    ++j;
-  }
   const GemmJob& J = a.job[j];
   const SplitX& x = a.x;
   const int M = x.M, K = x.K;
@@ -199,31 +212,15 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   const bool pair = a.pair != 0;
 
   // Two stages (a step's operands) alternate; the per-super-block tables of
-  // Q4_K alternate with the super-block.
-  // token rows [hi, lo][token], swizzled (ASwz), one array per stage: the
-  // compiler tells LDS arrays apart when it places the waits for its DMA
-  // loads, so reads of one stage do not wait for the DMA into the other
-  __shared__ __align__(16) _Float16 As0[2][kTM][64];
-  __shared__ __align__(16) _Float16 As1[2][kTM][64];
+  // Q4_K and Q6_K alternate with the super-block.
   auto as = [&](int st) -> _Float16(*)[kTM][64] { return st ? As1 : As0; };
-  // quants of a step, 16-byte chunks side by side over the rows (a wave's
-  // reads of one chunk are 512 consecutive bytes):
-  //  Q4_K [stage][h][row]: bytes 16 h .. + 16 of the row's 32;
-  //  else [stage][2 p + h][row]: unsigned bytes, inputs 8 h .. + 8 of slices
-  //  2 p and 2 p + 1 (slice: 16 inputs of the step)
-  constexpr int kChunks = kQ4 ? 2 : 4;
-  __shared__ __align__(16) U4 Bq[2][kChunks][kTN];
-  // Q4_K [table][step][row]: UnpackQ4's pairs of the step's two sub-blocks
-  __shared__ __align__(16) U2 S4[kQ4 ? 2 : 1][4][kQ4 ? kTN : 1];
-  __shared__ __align__(16) _Float16 Ss[kQ4 ? 2 : 1][2][kTM][8];  // Q4_K [table][hi, lo][token]: sub-block sums
-  __shared__ __align__(16) _Float16 Mn[kQ4 ? 2 : 1][kTN][8];     // Q4_K [table][row]: integer mins
-  __shared__ float2 Dd[kQ4 ? 2 : 1][kTN];                        // Q4_K [table][row]: d, -32 dmin
-  // Q6_K [4 table + step][row]: d * sc of the step's 4 slices; Q8_0
-  // [stage][row]: d of its 2 blocks
-  constexpr int kSc = kQ4 ? 1 : kQ6 ? 4 : 2;
-  __shared__ __align__(16) float Sc[kQ4 ? 1 : kQ6 ? 8 : 2][kQ4 ? 1 : kTN][kSc];
-
-  __shared__ __align__(16) float Is[kTM];  // 1 / s of the token rows
+  auto& Bq = L.Bq;
+  auto& S4 = L.S4;
+  auto& Ss = L.Ss;
+  auto& Mn = L.Mn;
+  auto& Dd = L.Dd;
+  auto& Sc = L.Sc;
+  auto& Is = L.Is;
 
   // The weight row this thread stages, as local row br, and the half bq of a
   // step (Q4_K: 16 of its 32 quant bytes; Q6_K: ql / qh bytes 16 bq .. + 16,
@@ -644,6 +641,38 @@ __global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
   }
 }
 
+// A launch over jobs of type QA, or of QA and QB (Q4_K and Q6_K: a layer's q, k
+// and v in one launch; as two launches on two streams they cost ~20 us of
+// cross-stream waits per layer).
+template <int QA, int QB, int kTM>
+__global__ __launch_bounds__(kThreads) void TGemmKernel(TiledArgs a) {
+  using LA = TileLds<QA, kTM>;
+  using LB = TileLds<QB, kTM>;
+  __shared__ __align__(16) _Float16 As0[2][kTM][64];
+  __shared__ __align__(16) _Float16 As1[2][kTM][64];
+  __shared__ __align__(16) uint8_t rest[sizeof(LA) > sizeof(LB) ? sizeof(LA) : sizeof(LB)];
+  // the tiles from tail_wg on in K parts: workgroup tail_wg + ts i + z takes
+  // part z of tile tail_wg + i
+  int wgi = static_cast<int>(blockIdx.x), zt = -1;
+  const int ts = a.tail_split;
+  if (ts > 1 && wgi >= a.tail_wg) {
+    const int u = wgi - a.tail_wg;
+    wgi = u / ts;
+    zt = u - wgi * ts;
+    wgi += a.tail_wg;
+  }
+  const int tm = wgi % a.tiles_m;
+  int nt = wgi / a.tiles_m, j = 0;
+  while (j + 1 < a.n_jobs && nt >= a.tiles[j]) {
+    nt -= a.tiles[j];
+    ++j;
+  }
+  if (QA == QB || a.job[j].w.type == QA)
+    TGemmTile<QA, kTM>(a, wgi, zt, tm, nt, j, As0, As1, *reinterpret_cast<LA*>(rest));
+  else
+    TGemmTile<QB, kTM>(a, wgi, zt, tm, nt, j, As0, As1, *reinterpret_cast<LB*>(rest));
+}
+
 // The tail tiles of a pair launch: y = silu(g) * u with g, u the sums of the
 // tile's K parts (added in part order, then scaled as the full tiles' sums
 // are), the full tiles' SwiGLU arithmetic. Workgroup (tile, y) takes tokens
@@ -697,8 +726,13 @@ void LaunchTiled(const TiledArgs& a, hipStream_t s) {
   for (int j = 0; j < a.n_jobs; ++j) tiles += a.tiles[j];
   const uint32_t type = a.job[0].w.type;
   RPG_CHECK(type == kQ4_K || type == kQ6_K || type == kQ8_0, "tiled gemm: weight type %u", type);
-  for (int j = 1; j < a.n_jobs + (a.pair ? 1 : 0); ++j)
-    RPG_CHECK(a.job[j].w.type == type, "tiled gemm: one weight type per launch");
+  bool mixed = false;
+  for (int j = 1; j < a.n_jobs + (a.pair ? 1 : 0); ++j) {
+    const uint32_t tj = a.job[j].w.type;
+    RPG_CHECK(tj == type || (!a.pair && TiledMixes(tj) && TiledMixes(type)), "tiled gemm: types %u and %u in one launch",
+              type, tj);
+    mixed = mixed || tj != type;
+  }
   RPG_CHECK(a.x.K % 256 == 0 && a.x.K >= 256, "tiled gemm: K = %d is not a multiple of 256", a.x.K);
   RPG_CHECK(a.tokens == TiledTokens(a.x.M) && a.tiles_m == CeilDiv(a.x.M, a.tokens), "tiled gemm: bad token tiles");
   RPG_CHECK(a.ksplit >= 1 && a.ksplit <= a.x.K / 256, "tiled gemm: bad K split %d", a.ksplit);
@@ -711,21 +745,26 @@ void LaunchTiled(const TiledArgs& a, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(total + n_tail * (a.tail_split - 1)), static_cast<unsigned>(a.ksplit));
   const bool small = a.tokens == 64;
   const dim3 block(kThreads);
-  if (type == kQ4_K) {
+  if (mixed) {
     if (small)
-      hipLaunchKernelGGL((TGemmKernel<kQ4_K, 64>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((TGemmKernel<kQ4_K, kQ6_K, 64>), grid, block, 0, s, a);
     else
-      hipLaunchKernelGGL((TGemmKernel<kQ4_K, 128>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((TGemmKernel<kQ4_K, kQ6_K, 128>), grid, block, 0, s, a);
+  } else if (type == kQ4_K) {
+    if (small)
+      hipLaunchKernelGGL((TGemmKernel<kQ4_K, kQ4_K, 64>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((TGemmKernel<kQ4_K, kQ4_K, 128>), grid, block, 0, s, a);
   } else if (type == kQ6_K) {
     if (small)
-      hipLaunchKernelGGL((TGemmKernel<kQ6_K, 64>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((TGemmKernel<kQ6_K, kQ6_K, 64>), grid, block, 0, s, a);
     else
-      hipLaunchKernelGGL((TGemmKernel<kQ6_K, 128>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((TGemmKernel<kQ6_K, kQ6_K, 128>), grid, block, 0, s, a);
   } else {
     if (small)
-      hipLaunchKernelGGL((TGemmKernel<kQ8_0, 64>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((TGemmKernel<kQ8_0, kQ8_0, 64>), grid, block, 0, s, a);
     else
-      hipLaunchKernelGGL((TGemmKernel<kQ8_0, 128>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((TGemmKernel<kQ8_0, kQ8_0, 128>), grid, block, 0, s, a);
   }
   HIP_CHECK(hipGetLastError());
   if (n_tail > 0) {

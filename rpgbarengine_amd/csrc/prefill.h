@@ -23,6 +23,7 @@
 
 #include <cstdint>
 
+#include "common.h"
 #include "kernels.h"
 
 namespace rpg {
@@ -70,6 +71,8 @@ struct GemmJob {
   int64_t ldy = 0;
   Epilogue epi = kStore;
 };
+// Whether jobs of two types share a QGemm launch.
+bool QGemmShares(const MatRef& a, const MatRef& b);
 // True when W can run on QGemm (K-quants need K a multiple of 256).
 bool QGemmSupports(const MatRef& w);
 // cus: the compute units the launch may count on (0: all), where another
@@ -99,6 +102,9 @@ void SwiGLURows(const float* g, const float* u, float* y, int64_t n, hipStream_t
 // 1.7B Q4_K_M 65 4.7 / 5.9, 300 6.2 / 7.5, 512 8.7 / 8.8).
 constexpr int kTiledRows = 256;
 inline int TiledTokens(int M) { return M <= 320 ? 64 : 128; }
+
+// The types a tiled launch may hold side by side (any other launch: one type).
+inline bool TiledMixes(uint32_t type) { return type == kQ4_K || type == kQ6_K; }
 
 struct TiledArgs {
   SplitX x;

@@ -1,17 +1,16 @@
 // Prefill projections on the gfx950 matrix cores (v_mfma_f32_16x16x32_f16);
 // the operand construction that keeps them exact is described in prefill.h.
 //
-// Kernels: QGemm4Kernel (Q4_K) and QGemm6Kernel (Q6_K), 4 waves over 32
-// tokens x 256 weight rows with per-super-block scale tables in LDS, and
-// QGemm8Kernel (Q8_0), 2 waves over 64 tokens x 128 rows. In all of them the
-// token operands of a 64-input step (both f16 parts) are staged in LDS once
-// for the workgroup, every lane assembles its weight operand from the raw
-// quant bytes, and the next step's loads are in flight while the current one
-// is multiplied.
+// The tiled GEMM (gemm_tiled.hip) takes every matrix whose width is a
+// multiple of 256. QGemm8Kernel here serves the other Q8_0 widths: 2 waves
+// over 64 tokens x 128 rows, the token operands of a 64-input step (both f16
+// parts) staged in LDS once for the workgroup, every lane assembling its
+// weight operand from the raw quant bytes, the next step's loads in flight
+// while the current one is multiplied.
 //
 // MFMA operand layout (16x16x32 f16): lane l holds A[i = l % 16][8*(l/16) ..
 // +8), B[8*(l/16) .. +8][j = l % 16]; the result C[4*(l/16) + e][l % 16],
-// e < 4. In the 16x16x16 form used for the Q4_K min term, 4 k per lane.
+// e < 4.
 
 #include <hip/hip_runtime.h>
 
@@ -555,6 +554,10 @@ bool TiledTakes(const MatRef& w) {
 }
 }  // namespace
 
+bool QGemmShares(const MatRef& a, const MatRef& b) {
+  return a.type == b.type || (TiledMixes(a.type) && TiledMixes(b.type) && TiledTakes(a) && TiledTakes(b));
+}
+
 bool QGemmSupports(const MatRef& w) {
   return ((w.type == kQ4_K || w.type == kQ6_K) && TiledTakes(w)) || (w.type == kQ8_0 && w.cols % 64 == 0);
 }
@@ -632,7 +635,7 @@ void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, Spli
   int64_t cols = 0;
   for (int j = 0; j < n_jobs; ++j) {
     RPG_CHECK(QGemmSupports(jobs[j].w) && jobs[j].w.cols == x.K, "qgemm: unsupported matrix");
-    RPG_CHECK(jobs[j].w.type == jobs[0].w.type, "qgemm: one weight type per launch");
+    RPG_CHECK(QGemmShares(jobs[j].w, jobs[0].w), "qgemm: types %u and %u in one launch", jobs[0].w.type, jobs[j].w.type);
     pcol[j] = static_cast<int32_t>(cols);
     cols += jobs[j].w.rows;
   }
