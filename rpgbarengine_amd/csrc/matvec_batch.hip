@@ -727,6 +727,20 @@ int FewTokenLimit() {
   return limit;
 }
 
+// Per million weights, the matvec takes about 0.19 us a group of 8 tokens
+// (0.25 for Q8_0; 0.39 for a Q6_K matrix, whose wide inputs make groups of 4)
+// beside 6 us; the GEMM, its operand split included, 0.25 us (0.5, 0.4) up to
+// 64 tokens beside 22 us (25). Measured, matvec / GEMM, us: 37 tokens, 4B
+// gate+up (49.8 M weights) 53 / 35, down (24.9 M) Q4_K 33 / 32, Q6_K 55 / 39,
+// QKV (15.7 M) 27 / 26, O (10.5 M) 18 / 23; 48 tokens, 1.7B Q8_0 gate+up
+// (25.2 M) 44 / 37, down (12.6 M) 31 / 32.
+bool FewTokensWin(int64_t weights, uint32_t type, int n) {
+  if (std::getenv("RPG_FEW_TOKENS") != nullptr) return true;  // (a sweep's limit alone decides)
+  const bool q6 = type == kQ6_K, q8 = type == kQ8_0;
+  const double w = static_cast<double>(weights) * 1e-6, groups = static_cast<double>(CeilDiv(n, 8));
+  return 6.0 + (q6 ? 0.39 : q8 ? 0.25 : 0.19) * w * groups <= (q8 ? 25.0 : 22.0) + (q6 ? 0.4 : q8 ? 0.5 : 0.25) * w;
+}
+
 namespace {
 
 int ComputeUnits() {
