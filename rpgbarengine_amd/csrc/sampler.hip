@@ -942,7 +942,7 @@ __device__ __forceinline__ bool TopKMode(const SamplerParamsDev& P, int n) {
 }
 
 // Rows drawn by the full-vocabulary kernels below: sampled, no top-k filter, and a vocabulary
-// whose per-row scratch fits (WideRowBytesA / B below).
+// whose per-row scratch fits (WideRowBytesA, kWideRowBytesB below).
 __device__ __host__ __forceinline__ bool WideVocab(int n) { return n >= 16384; }
 __device__ __forceinline__ bool WideMode(const SamplerParamsDev& P, int n) {
   return P.temperature > 0.0f && !TopKMode(P, n) && WideVocab(n);
@@ -1114,12 +1114,12 @@ __global__ __launch_bounds__(kThreads) void SampleKernel(Ctx c, int n_slices, in
 //   exp      e = expf(s - max), slice double sums
 //   norm     inv = float(1 / sum) (bounded parallel sum, else sequential),
 //            p = e * inv into a second buffer (a sequential fallback of
-//            another workgroup may still read e); top-p radix pass 0 slice
-//            histograms (count and exact 2^-57 fixed-point mass: order-free
-//            integer sums)
-//   radix    passes 1..3: the previous pass's selection from its summed
-//            histograms (slice 0 records it for the next launch), then this
-//            pass's histograms
+//            another workgroup may still read e); top-p radix pass 0: the
+//            slice's histogram (count and exact 2^-57 fixed-point mass) added
+//            to the row's (order-free integer sums)
+//   radix    passes 1, 2: the previous pass's selection from its histogram
+//            (slice 0 records it for the next launch), then this pass's
+//            histogram
 //   cut      (one workgroup per row) the last selection: vstar and the tie
 //            count J the reference zeroes; a tie set straddling the cut
 //            replays the reference's sort (TieOrder), which zeroes its first J
@@ -1136,7 +1136,17 @@ __global__ __launch_bounds__(kThreads) void SampleKernel(Ctx c, int n_slices, in
 // row whose survivors are the whole vocabulary, with the same arithmetic.
 // ---------------------------------------------------------------------------
 
-constexpr int kRadixPasses = 4;
+// The radix digits of a key, from the top: 11, 11 and 10 bits. (Four 8-bit
+// passes whose every workgroup summed the 38 slices' histograms itself, 117
+// KB, took 15.6 us each; one pass fewer and one histogram per row, to which
+// the slices add their nonzero bins with device-scope atomics, 3 x 15.6 -> 2
+// x 7 us for one row of 151936.)
+constexpr int kRadixPasses = 3;
+constexpr int kRadixMaxBins = 2048;
+__host__ __device__ constexpr int RadixShift(int pass) { return pass == 0 ? 21 : pass == 1 ? 10 : 0; }
+__host__ __device__ constexpr int RadixBins(int pass) { return pass == 2 ? 1024 : 2048; }
+__host__ __device__ constexpr int RadixOffset(int pass) { return 2048 * pass; }
+constexpr int kRadixAllBins = 2048 + 2048 + 1024;
 constexpr int kPer = kSlice / kSelThreads;  // elements per thread of a slice
 
 // Whole-row results that later launches read, each written by one workgroup.
@@ -1168,8 +1178,8 @@ struct WideRow {
   int32_t* stiny;             // [S] a nonzero p2 < 2^-29 in the slice
   int32_t* sexp;              // [S] smallest exponent field of a nonzero e in the slice (255: none)
   int32_t* sexp2;             // [S] the same for the cut p
-  uint32_t* hcnt;             // [pass][S][256]
-  unsigned long long* hmass;  // [pass][S][256]
+  uint32_t* hcnt;             // the passes' bins (RadixOffset): counts, cleared by the exp launch
+  unsigned long long* hmass;  // masses
 };
 
 constexpr size_t kWideStateBytes = (sizeof(WideState) + 15) & ~static_cast<size_t>(15);
@@ -1204,13 +1214,13 @@ __device__ __forceinline__ WideRow WideView(const Ctx& c, int row, int S) {
   uint8_t* b = reinterpret_cast<uint8_t*>(c.cand_i + static_cast<int64_t>(row) * c.n);
   b = reinterpret_cast<uint8_t*>((reinterpret_cast<uintptr_t>(b) + 15) & ~static_cast<uintptr_t>(15));
   w.hmass = reinterpret_cast<unsigned long long*>(b);
-  w.hcnt = reinterpret_cast<uint32_t*>(b + static_cast<size_t>(8) * kRadixPasses * S * 256);
+  w.hcnt = reinterpret_cast<uint32_t*>(b + static_cast<size_t>(8) * kRadixAllBins);
   return w;
 }
 
 // Bytes of each of the two regions a row needs (checked on the host).
 __host__ __device__ constexpr size_t WideRowBytesA(int S) { return 16 + kWideStateBytes + 52 * static_cast<size_t>(S); }
-__host__ __device__ constexpr size_t WideRowBytesB(int S) { return 16 + 12 * static_cast<size_t>(kRadixPasses) * S * 256; }
+constexpr size_t kWideRowBytesB = 16 + 12 * static_cast<size_t>(kRadixAllBins);
 
 using WSh = Shared<kSelThreads>;
 
@@ -1271,8 +1281,15 @@ __global__ __launch_bounds__(kSelThreads) void WideExpKernel(Ctx c) {
     const int i = SliceElem(slice, t, n);
     v[t] = i >= 0 ? work[i] : 0.0f;
   }
-  float mx = w.smax[0];
-  for (int q = 1; q < S; ++q) mx = fmaxf(mx, w.smax[q]);
+  // (this launch's share of the row's radix histograms, empty before the norm
+  // launch adds to them)
+  for (int b = slice * kSelThreads + static_cast<int>(threadIdx.x); b < kRadixAllBins; b += S * kSelThreads) {
+    w.hcnt[b] = 0;
+    w.hmass[b] = 0;
+  }
+  float mx = -__builtin_inff();
+  for (int q = static_cast<int>(threadIdx.x & 63); q < S; q += 64) mx = fmaxf(mx, w.smax[q]);
+  mx = lanes::WaveMaxF(mx);
   double part = 0.0;
 #pragma unroll
   for (int t = 0; t < kPer; ++t) {
@@ -1327,12 +1344,17 @@ __device__ double SequentialSum(const float* vals, int n, float* buf) {
 __device__ float WideInv(const double* ssum, const int32_t* sexp, int S, const float* vals, int n, int slice, WSh& sh,
                          unsigned long long* fallbacks) {
   __shared__ float buf[kSlice];
+  // the slice sums in slice order: a lane per slice loads them, one after
+  // another they are added
   double T = 0.0;
   int E = 255;
-  for (int q = 0; q < S; ++q) {
-    T += ssum[q];
-    E = min(E, sexp[q]);
+  for (int q0 = 0; q0 < S; q0 += 64) {
+    const int q = q0 + static_cast<int>(threadIdx.x & 63), m = min(64, S - q0);
+    const double mine = q < S ? ssum[q] : 0.0;
+    if (q < S) E = min(E, sexp[q]);
+    for (int i = 0; i < m; ++i) T += lanes::ReadLaneD(mine, i);
   }
+  E = WaveReduce(E, [](int x, int y) { return min(x, y); });
   // Every value is a multiple of the quantum 2^(E - 150) (2^-149 for a
   // subnormal, E = 0): when the total stays below 2^53 quanta every partial
   // sum, in any order, is exact in double, so the parallel sum is the
@@ -1357,15 +1379,26 @@ __device__ __forceinline__ unsigned long long TopPThreshold(const SamplerParamsD
   return static_cast<unsigned long long>((1.0 - static_cast<double>(P.top_p)) * 0x1p57);
 }
 
+// LDS of a radix pass: a slice's histogram, the selection.
+struct WideBins {
+  alignas(16) unsigned long long mass[kRadixMaxBins];
+  uint32_t cnt[kRadixMaxBins];
+};
+struct WidePick {
+  unsigned long long wave[kThreads / 64], cum;
+  uint32_t sel, cnt;
+  int32_t flag;
+};
+
 // This slice's histogram of radix pass `pass` over p[] (values held by the
-// thread, v[t] for element t) with keys matching (prefix, mask): count and
-// 2^-57 fixed-point mass per 8-bit bin.
-__device__ void WideHistogram(const WideRow& w, const float (&v)[kPer], int n, int slice, int S, int pass,
-                              uint32_t prefix, uint32_t mask, WSh& sh) {
-  const int shift = 24 - 8 * pass;
-  for (int b = threadIdx.x; b < 256; b += kSelThreads) {
-    sh.cnt[b] = 0;
-    sh.mass[b] = 0;
+// thread, v[t] for element t) with keys matching (prefix, mask), added to the
+// row's: count and 2^-57 fixed-point mass per bin.
+__device__ void WideHistogram(const WideRow& w, const float (&v)[kPer], int n, int slice, int pass, uint32_t prefix,
+                              uint32_t mask, WideBins& h) {
+  const int shift = RadixShift(pass), bins = RadixBins(pass);
+  for (int b = threadIdx.x; b < bins; b += kSelThreads) {
+    h.cnt[b] = 0;
+    h.mass[b] = 0;
   }
   __syncthreads();
 #pragma unroll
@@ -1374,43 +1407,63 @@ __device__ void WideHistogram(const WideRow& w, const float (&v)[kPer], int n, i
     const uint32_t key = __float_as_uint(v[t]);
     const bool act = i >= 0 && (key & mask) == prefix;
     const unsigned long long mj = act ? static_cast<unsigned long long>(static_cast<double>(v[t]) * 0x1p57) : 0ull;
-    AggAdd(sh.cnt, sh.mass, act, (key >> shift) & 255u, mj);
+    AggAdd(h.cnt, h.mass, act, (key >> shift) & static_cast<uint32_t>(bins - 1), mj);
   }
   __syncthreads();
-  const size_t o = (static_cast<size_t>(pass) * S + slice) * 256;
-  for (int b = threadIdx.x; b < 256; b += kSelThreads) {
-    w.hcnt[o + b] = sh.cnt[b];
-    w.hmass[o + b] = sh.mass[b];
+  const int o = RadixOffset(pass);
+  for (int b = threadIdx.x; b < bins; b += kSelThreads) {
+    if (h.cnt[b] == 0) continue;
+    __hip_atomic_fetch_add(&w.hcnt[o + b], h.cnt[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (h.mass[b] != 0)
+      __hip_atomic_fetch_add(&w.hmass[o + b], h.mass[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
 // Radix pass `pass`'s selection, as FinishHead's pass makes it, from its
-// slice histograms (summed over the slices: exact) and the state after the
-// previous pass (in: prefix, mask, cum). Every thread returns the new state;
-// the return value is the "no bin crosses" flag.
+// histogram and the state after the previous pass (in: prefix, mask, cum):
+// the first bin b with cum + the mass of bins 0 .. b above THR. Every thread
+// returns the new state; the return value is the "no bin crosses" flag.
 template <int NT>
-__device__ int WideSelect(const WideRow& w, int S, int pass, unsigned long long THR, uint32_t* prefix, uint32_t* mask,
-                          unsigned long long* cum, uint32_t* cnt_sel, Shared<NT>& sh) {
-  const int shift = 24 - 8 * pass;
-  for (int b = threadIdx.x; b < 256; b += NT) {
-    uint32_t cs = 0;
-    unsigned long long ms = 0;
-    for (int q = 0; q < S; ++q) {
-      const size_t o = (static_cast<size_t>(pass) * S + q) * 256 + b;
-      cs += w.hcnt[o];
-      ms += w.hmass[o];
+__device__ int WideSelect(const WideRow& w, int pass, unsigned long long THR, uint32_t* prefix, uint32_t* mask,
+                          unsigned long long* cum, uint32_t* cnt_sel, WidePick& pk) {
+  constexpr int kMaxPer = kRadixMaxBins / NT;
+  const int shift = RadixShift(pass), o = RadixOffset(pass), per = RadixBins(pass) / NT;
+  const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6;
+  unsigned long long mb[kMaxPer], mine = 0;
+#pragma unroll
+  for (int i = 0; i < kMaxPer; ++i) mb[i] = i < per ? w.hmass[o + per * tid + i] : 0ull;
+#pragma unroll
+  for (int i = 0; i < kMaxPer; ++i) mine += mb[i];
+  const unsigned long long incl = lanes::WaveInclusiveAdd(mine);
+  if ((tid & 63) == 63) pk.wave[wave] = incl;
+  if (tid == 0) pk.flag = 1;
+  __syncthreads();
+  unsigned long long below = *cum + incl - mine;  // the mass below this thread's bins
+  for (int q = 0; q < wave; ++q) below += pk.wave[q];
+  if (below <= THR && below + mine > THR) {  // (one thread)
+    int sel = per - 1;
+#pragma unroll
+    for (int i = 0; i < kMaxPer; ++i) {
+      if (i < per - 1 && sel == per - 1) {
+        if (below + mb[i] > THR)
+          sel = i;
+        else
+          below += mb[i];
+      }
     }
-    sh.cnt[b] = cs;
-    sh.mass[b] = ms;
+    pk.sel = static_cast<uint32_t>(per * tid + sel);
+    pk.cum = below;
+    pk.cnt = w.hcnt[o + per * tid + sel];
+    pk.flag = 0;
   }
   __syncthreads();
-  if (threadIdx.x < 64) SelectBinAsc(sh.mass, *cum, THR, &sh.sel, &sh.u[0], &sh.flag);
-  __syncthreads();
-  const int all_zero = sh.flag;
-  *cum = sh.u[0];
-  *prefix |= sh.sel << shift;
-  *mask |= 0xFFu << shift;
-  *cnt_sel = sh.cnt[sh.sel];
+  const int all_zero = pk.flag;
+  if (!all_zero) {
+    *cum = pk.cum;
+    *prefix |= pk.sel << shift;
+    *mask |= static_cast<uint32_t>(RadixBins(pass) - 1) << shift;
+    *cnt_sel = pk.cnt;
+  }
   __syncthreads();
   return all_zero;
 }
@@ -1435,6 +1488,7 @@ __device__ __forceinline__ bool WideStateAfter(const WideRow& w, int pass, uint3
 // norm: inv, p, radix pass 0
 __global__ __launch_bounds__(kSelThreads) void WideNormKernel(Ctx c) {
   __shared__ WSh sh;
+  __shared__ WideBins hist;
   const int row = blockIdx.y, slice = blockIdx.x, n = c.n, S = gridDim.x;
   const SamplerParamsDev P = c.params[row];
   if (!WideMode(P, n)) return;
@@ -1455,13 +1509,14 @@ __global__ __launch_bounds__(kSelThreads) void WideNormKernel(Ctx c) {
     if (i >= 0) pb[i] = v[t];
   }
   if (!TopPActive(P)) return;
-  WideHistogram(w, v, n, slice, S, 0, 0u, 0u, sh);
+  WideHistogram(w, v, n, slice, 0, 0u, 0u, hist);
 }
 
-// radix pass `pass` (1..3): the previous pass's selection, then this pass's
-// histograms
+// radix pass `pass` (1, 2): the previous pass's selection, then this pass's
+// histogram
 __global__ __launch_bounds__(kSelThreads) void WideRadixKernel(Ctx c, int pass) {
-  __shared__ WSh sh;
+  __shared__ WideBins hist;
+  __shared__ WidePick pick;
   const int row = blockIdx.y, slice = blockIdx.x, n = c.n, S = gridDim.x;
   const SamplerParamsDev P = c.params[row];
   if (!WideMode(P, n) || !TopPActive(P)) return;
@@ -1473,13 +1528,13 @@ __global__ __launch_bounds__(kSelThreads) void WideRadixKernel(Ctx c, int pass) 
     const int i = SliceElem(slice, t, n);
     v[t] = i >= 0 ? pb[i] : 0.0f;
   }
-  uint32_t prefix, mask, cnt;
+  uint32_t prefix, mask, cnt = 0;
   unsigned long long cum;
   if (!WideStateAfter(w, pass - 2, &prefix, &mask, &cum)) {
     if (slice == 0 && threadIdx.x == 0) w.st->all_zero[pass - 1] = 1;  // carried to the later passes
     return;
   }
-  const int all_zero = WideSelect(w, S, pass - 1, TopPThreshold(P), &prefix, &mask, &cum, &cnt, sh);
+  const int all_zero = WideSelect<kSelThreads>(w, pass - 1, TopPThreshold(P), &prefix, &mask, &cum, &cnt, pick);
   if (slice == 0 && threadIdx.x == 0) {
     w.st->prefix[pass - 1] = prefix;
     w.st->mask[pass - 1] = mask;
@@ -1488,13 +1543,14 @@ __global__ __launch_bounds__(kSelThreads) void WideRadixKernel(Ctx c, int pass) 
     w.st->cnt_sel[pass - 1] = cnt;
   }
   if (all_zero) return;
-  WideHistogram(w, v, n, slice, S, pass, prefix, mask, sh);
+  WideHistogram(w, v, n, slice, pass, prefix, mask, hist);
 }
 
 // cut: one 1024-thread workgroup per row
 __global__ __launch_bounds__(kThreads) void WideCutKernel(Ctx c) {
   __shared__ Shared<kThreads> sh;
   __shared__ TieShared ts;
+  __shared__ WidePick pick;
   const int row = blockIdx.x, n = c.n, S = (n + kSlice - 1) / kSlice;
   const SamplerParamsDev P = c.params[row];
   if (!WideMode(P, n)) return;
@@ -1504,10 +1560,10 @@ __global__ __launch_bounds__(kThreads) void WideCutKernel(Ctx c) {
     return;
   }
   const unsigned long long THR = TopPThreshold(P);
-  uint32_t prefix, mask, ties;
+  uint32_t prefix, mask, ties = 0;
   unsigned long long cum;
   if (!WideStateAfter(w, kRadixPasses - 2, &prefix, &mask, &cum) ||
-      WideSelect(w, S, kRadixPasses - 1, THR, &prefix, &mask, &cum, &ties, sh)) {
+      WideSelect<kThreads>(w, kRadixPasses - 1, THR, &prefix, &mask, &cum, &ties, pick)) {
     if (threadIdx.x == 0) w.st->mode = 1;
     return;
   }
@@ -1686,28 +1742,41 @@ __global__ __launch_bounds__(kSelThreads) void WideDrawKernel(Ctx c) {
   const float* work = c.work + static_cast<int64_t>(row) * n;
   const uint64_t pos = c.counter_dev ? static_cast<uint64_t>(c.counter_dev[row]) : static_cast<uint64_t>(c.counter_host);
   const float u = CounterUniform(P.seed, pos);
+  // a lane per slice reads its figures (each wave for itself)
   int tiny = 0;
-  for (int q = 0; q < S; ++q) tiny |= w.stiny[q];
+  for (int q = static_cast<int>(threadIdx.x & 63); q < S; q += 64) tiny |= w.stiny[q];
+  tiny = __ballot(tiny != 0) != 0 ? 1 : 0;
   int ans = -1;
   if (!tiny) {
     // exact: every partial sum is a multiple of 2^-52 below 2
     const unsigned long long U = static_cast<unsigned long long>(static_cast<double>(u) * 0x1p52);
     unsigned long long cum = 0;
     int hit = -1;
-    for (int q = 0; q < S; ++q) {
-      if (cum + w.smass[q] > U) {
-        hit = q;
-        break;
+    for (int q0 = 0; q0 < S && hit < 0; q0 += 64) {
+      const int q = q0 + static_cast<int>(threadIdx.x & 63);
+      const unsigned long long m = q < S ? w.smass[q] : 0ull;
+      const unsigned long long incl = lanes::WaveInclusiveAdd(m);
+      const unsigned long long over = __ballot(cum + incl > U);
+      if (over != 0) {
+        const int l = __ffsll(static_cast<long long>(over)) - 1;
+        hit = q0 + l;
+        cum += lanes::ReadLaneT(incl - m, l);
+      } else {
+        cum += lanes::ReadLaneT(incl, 63);
       }
-      cum += w.smass[q];
     }
     if (hit >= 0) {
       // the slice in index order: thread t takes elements kPer t .. kPer t + kPer
       const int i0 = hit * kSlice, m = min(kSlice, n - i0);
       const int b = i0 + min(m, static_cast<int>(threadIdx.x) * kPer);
       const int e = i0 + min(m, (static_cast<int>(threadIdx.x) + 1) * kPer);
+      float v[kPer];  // (every load before the first use)
+#pragma unroll
+      for (int t = 0; t < kPer; ++t) v[t] = work[min(b + t, i0 + m - 1)];
       unsigned long long mine = 0;
-      for (int i = b; i < e; ++i) mine += static_cast<unsigned long long>(static_cast<double>(work[i]) * 0x1p52);
+#pragma unroll
+      for (int t = 0; t < kPer; ++t)
+        if (b + t < e) mine += static_cast<unsigned long long>(static_cast<double>(v[t]) * 0x1p52);
       const unsigned long long incl = lanes::WaveInclusiveAdd(mine);
       __syncthreads();
       if ((threadIdx.x & 63) == 63) sh.u[threadIdx.x >> 6] = incl;
@@ -1716,12 +1785,10 @@ __global__ __launch_bounds__(kSelThreads) void WideDrawKernel(Ctx c) {
       for (int q = 0; q < static_cast<int>(threadIdx.x >> 6); ++q) run += sh.u[q];
       run += incl - mine;
       int found = 0x7fffffff;
-      for (int i = b; i < e; ++i) {
-        run += static_cast<unsigned long long>(static_cast<double>(work[i]) * 0x1p52);
-        if (run > U) {
-          found = i;
-          break;
-        }
+#pragma unroll
+      for (int t = 0; t < kPer; ++t) {
+        if (b + t < e) run += static_cast<unsigned long long>(static_cast<double>(v[t]) * 0x1p52);
+        if (b + t < e && run > U && found == 0x7fffffff) found = b + t;
       }
       found = BlockMinI(found, sh);
       if (found != 0x7fffffff) ans = found;
@@ -1938,7 +2005,7 @@ void Sampler::Enqueue(const float* logits, int64_t ld, const int32_t* counter, i
   // a row's scratch: the small arrays in its cand_v slot, the histograms in
   // its cand_i slot (each 4 * vocab bytes, 4-byte aligned)
   RPG_CHECK(!wide || (WideRowBytesA(n_slices) + 16 <= 4 * static_cast<size_t>(vocab_) &&
-                      WideRowBytesB(n_slices) + 16 <= 4 * static_cast<size_t>(vocab_)),
+                      kWideRowBytesB + 16 <= 4 * static_cast<size_t>(vocab_)),
             "sampler: vocabulary %d too small for the full-vocabulary kernels", vocab_);
   const dim3 grid(static_cast<unsigned>(n_slices), static_cast<unsigned>(rows_));
   hipLaunchKernelGGL(TopKSelectKernel, grid, dim3(kSelThreads), 0, s, c, wide);

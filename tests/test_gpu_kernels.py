@@ -408,6 +408,21 @@ def test_sampler_full_vocabulary_extremes(case):
         assert tok == oracle.sample_token(logits, temperature, 0, top_p, u), trial
 
 
+@pytest.mark.parametrize("vocab", [16384, 16385, 69632, 262144])
+@pytest.mark.parametrize("top_p", [0.0, 0.3, 0.95])
+def test_sampler_full_vocabulary_sizes(vocab, top_p):
+    """The full-vocabulary draw at its smallest row, slices of one logit, and
+    64 slices (a wave's lanes): bitwise probs and the same token as the
+    reference."""
+    rng = np.random.default_rng(vocab)
+    logits = (rng.standard_normal(vocab) * 1.7).astype(np.float32)
+    u = oracle.counter_uniform(9, 21)
+    tok, probs = eng.sample(logits, 0.8, 0, top_p, 9, 21, want_probs=True)
+    want_p = oracle.filter_to_probs(logits, 0.8, 0, top_p)
+    assert np.array_equal(probs.view(np.uint32), want_p.view(np.uint32))
+    assert tok == oracle.sample_token(logits, 0.8, 0, top_p, u)
+
+
 def _straddle_case(rng, vocab, top_k, temperature, group):
     """Logits with `group` equal values placed where the top-p cut falls in
     the middle of them: returns (logits, top_p)."""
