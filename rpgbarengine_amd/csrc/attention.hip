@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "expf_glibc.h"
@@ -153,6 +154,14 @@ __global__ __launch_bounds__(128) void DecodeCombineKernel(AttnArgs a, int n_spl
 // probabilities are a B operand of O^T = V^T.P^T as they stand, keys taken
 // in slot order 8 g + 4 jt + e. V^T rows are staged in that slot order.
 constexpr int kQB = 16;        // queries per query tile (one tile per workgroup, or two: PrefillKernel)
+// Query blocks from which the key blocks are converted to f16 once, by a
+// launch of their own, instead of by every query block that walks them: the
+// conversion took more issue slots than the products (~400 VALU instructions
+// per wave and step of 64 keys against 48 MFMAs). Per layer, us, before / after
+// (conversion included): 3999 tokens of the 1.7B shape 477 / 374, 512 of the 4B
+// 36 / 32, 203 behind 1500 60 / 55; at fewer query blocks the launch (5 - 10 us)
+// costs what it saves.
+constexpr int kImageQueryBlocks = 6;
 constexpr int kWideQueries = 1024;  // segments at least this long take two query tiles per workgroup (G <= 2)
 constexpr int kKB = 32;        // keys per block
 constexpr int kKH = kHd + 8;   // K row in LDS (halfs)
@@ -210,14 +219,88 @@ __device__ __forceinline__ F4v Mfma16x3(H8v ah, H8v al, H8v bh, H8v bl, F4v c) {
   return Mfma16(al, bh, Mfma16(ah, bl, Mfma16(ah, bh, c)));
 }
 
+// A 32-key block of the cache as the f16 operands a step stages: K [hi, lo]
+// [key][dimension], V^T [hi, lo][dimension][slot], then the inverse scales of
+// the keys and of the value dimensions.
+constexpr int kImgHalfs = 2 * kKB * kHd;  // each of K and V^T
+constexpr int kImgFloats = kImgHalfs + kKB + kHd;
+
+// K unit: 4 dimensions at 4 c4 of key j (32 adjacent lanes hold a key row):
+// scaled, split.
+__device__ __forceinline__ void SplitKUnit(F4v x, H4v* hi, H4v* lo, float* inv) {
+  float mx = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+  const int se = ScaleExp(Max32Lanes(mx));
+  const float sk = Pow2(se);
+  *inv = Pow2(-se);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) SplitHalf(x[e] * sk, *hi, *lo, e);
+}
+// V unit, one dimension of it: 4 consecutive keys x (a dimension's 32 keys sit
+// in 8 adjacent lanes).
+__device__ __forceinline__ void SplitVUnit(F4v x, H4v* hi, H4v* lo, float* inv) {
+  float mx = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+  const int se = ScaleExp(Max8Lanes(mx));
+  const float sv = Pow2(se);
+  *inv = Pow2(-se);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) SplitHalf(x[r] * sv, *hi, *lo, r);
+}
+// Keys 4 jq .. + 3 of a block in V^T slot order.
+__device__ __forceinline__ int VSlot(int jq) { return jq < 4 ? 8 * jq : 8 * (jq - 4) + 4; }
+
+// The images of every key block of the segment's history: grid (kv head,
+// block), 256 threads. Keys past the last one repeat it.
+__global__ __launch_bounds__(256) void KvImageKernel(AttnArgs a, int n_keys) {
+  const int kh = blockIdx.x, blk = blockIdx.y, tid = threadIdx.x;
+  const float* kb = a.kcache + static_cast<int64_t>(kh) * a.max_seq * kHd;
+  const float* vb = a.vcache + static_cast<int64_t>(kh) * a.max_seq * kHd;
+  float* img = a.image + (static_cast<int64_t>(kh) * gridDim.y + blk) * kImgFloats;
+  _Float16* ki = reinterpret_cast<_Float16*>(img);
+  _Float16* vi = ki + kImgHalfs;
+  float* inv = img + kImgHalfs;
+  F4v kr[4], vr[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int u = tid + 256 * i, c4 = u & 31, j = u >> 5;
+    kr[i] = *(const __attribute__((address_space(1))) F4v*)(kb + static_cast<int64_t>(min(blk * kKB + j, n_keys - 1)) *
+                                                                      kHd + 4 * c4);
+  }
+  const int jq = tid & 7, vc = tid >> 3;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    vr[r] = *(const __attribute__((address_space(1))) F4v*)(vb + static_cast<int64_t>(min(blk * kKB + 4 * jq + r,
+                                                                                          n_keys - 1)) * kHd + 4 * vc);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int u = tid + 256 * i, c4 = u & 31, j = u >> 5;
+    H4v hi, lo;
+    float s;
+    SplitKUnit(kr[i], &hi, &lo, &s);
+    *reinterpret_cast<H4v*>(ki + j * kHd + 4 * c4) = hi;
+    *reinterpret_cast<H4v*>(ki + (kKB + j) * kHd + 4 * c4) = lo;
+    if (c4 == 0) inv[j] = s;
+  }
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    H4v hi, lo;
+    float s;
+    SplitVUnit(F4v{vr[0][d], vr[1][d], vr[2][d], vr[3][d]}, &hi, &lo, &s);
+    const int dim = 4 * vc + d;
+    *reinterpret_cast<H4v*>(vi + dim * kKB + VSlot(jq)) = hi;
+    *reinterpret_cast<H4v*>(vi + (kHd + dim) * kKB + VSlot(jq)) = lo;
+    if (jq == 0) inv[kKB + dim] = s;
+  }
+}
+
 // G: query heads per KV head. Two waves per head split the key blocks (even
 // and odd) and merge their online-softmax states at the end; QT query tiles
 // of 16 share the workgroup's staged K/V blocks (long segments at G <= 2:
 // half the staging per query), so a workgroup has 2 G QT waves. With
 // gridDim.z = S > 1, workgroup z takes the z-th of S ranges of the block's
 // key steps and leaves its state to MergePrefillKernel (a.part: the output
-// sums [z][query][head][128], then (m, l) [z][query][head]).
-template <int G, int QT>
+// sums [z][query][head][128], then (m, l) [z][query][head]). kImg: the blocks
+// are staged from their images (KvImageKernel) instead of from the cache.
+template <int G, int QT, bool kImg>
 __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   constexpr int nt = 128 * G * QT;
   // halfs of one K block ([hi, lo][key][dimension]) and of one V^T block
@@ -280,8 +363,30 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   constexpr int kKPer = (kKUnits + nt - 1) / nt, kVPer = (kVUnits + nt - 1) / nt;
   // (native vectors: copies of HIP's float4 class stay memcpys that can keep
   // the registers in scratch memory)
-  F4v kreg[kKPer], vreg[kVPer][4];
+  F4v kreg[kImg ? 1 : kKPer], vreg[kImg ? 1 : kVPer][4];
+  // kImg: 16-byte units of the step's two images, thread tid takes u = tid +
+  // i * nt (block u / 2048, K part, key, chunk of 8 dimensions, then V^T
+  // part, dimension, chunk of 8 slots), and the scales as float4
+  constexpr int kIUnits = kBS * 2 * kImgHalfs / 8, kIPer = (kIUnits + nt - 1) / nt;
+  constexpr int kSUnits = kBS * (kKB + kHd) / 4;
+  static_assert(kSUnits <= nt, "a thread per four scales");
+  F4v ireg[kImg ? kIPer : 1], sreg = F4v{0.f, 0.f, 0.f, 0.f};
+  const float* img = kImg ? a.image + static_cast<int64_t>(kh) * a.image_blocks * kImgFloats : nullptr;
   auto load_step = [&](int st) {
+    if constexpr (kImg) {
+#pragma unroll
+      for (int i = 0; i < kIPer; ++i) {
+        const int u = min(tid + i * nt, kIUnits - 1);
+        const float* p = img + static_cast<int64_t>(min(kBS * st + (u >> 11), n_blocks - 1)) * kImgFloats;
+        ireg[i] = *(const __attribute__((address_space(1))) F4v*)(p + 4 * (u & 2047));
+      }
+      if (tid < kSUnits) {
+        const int bb = tid / (kSUnits / kBS), q = tid % (kSUnits / kBS);
+        sreg = *(const __attribute__((address_space(1))) F4v*)(
+            img + static_cast<int64_t>(min(kBS * st + bb, n_blocks - 1)) * kImgFloats + kImgHalfs + 4 * q);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < kKPer; ++i) {
       const int u = min(tid + i * nt, kKUnits - 1), c4 = u & 31, j = (u >> 5) & (kKB - 1), bb = u >> 10;
@@ -331,39 +436,44 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   }
   for (int st = st0; st < n_steps; ++st) {
     __syncthreads();  // the previous step's LDS reads are done
+    if constexpr (kImg) {
 #pragma unroll
-    for (int i = 0; i < kKPer; ++i) {
+      for (int i = 0; i < kIPer; ++i) {
+        const int u = tid + i * nt, bb = u >> 11, r = u & 1023;
+        if (kIUnits % nt != 0 && u >= kIUnits) break;
+        _Float16* p = (u & 1024) == 0
+                          ? kv + bb * kKbH + (r >> 9) * kKB * kKH + ((r >> 4) & 31) * kKH + 8 * (r & 15)
+                          : kv + kBS * kKbH + bb * kVbH + (r >> 9) * kHd * kVH + ((r >> 2) & 127) * kVH + 8 * (r & 3);
+        *reinterpret_cast<F4v*>(p) = ireg[i];
+      }
+      if (tid < kSUnits) {
+        const int bb = tid / (kSUnits / kBS), q = tid % (kSUnits / kBS);
+        *reinterpret_cast<F4v*>(q < kKB / 4 ? &kinv[bb][4 * q] : &vinv[bb][4 * q - kKB]) = sreg;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < (kImg ? 0 : kKPer); ++i) {
       const int u = tid + i * nt, c4 = u & 31, j = (u >> 5) & (kKB - 1), bb = u >> 10;
       if (kKUnits % nt != 0 && u >= kKUnits) break;
-      // the key row's scale (its 32 column chunks sit in 32 adjacent lanes)
-      float mx = fmaxf(fmaxf(fabsf(kreg[i][0]), fabsf(kreg[i][1])), fmaxf(fabsf(kreg[i][2]), fabsf(kreg[i][3])));
-      const int se = ScaleExp(Max32Lanes(mx));
-      const float sk = Pow2(se);
-      if (c4 == 0) kinv[bb][j] = Pow2(-se);
       _Float16* ks = kv + bb * kKbH + j * kKH + 4 * c4;
       H4v hi, lo;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) SplitHalf(kreg[i][e] * sk, hi, lo, e);
+      float inv;
+      SplitKUnit(kreg[i], &hi, &lo, &inv);
+      if (c4 == 0) kinv[bb][j] = inv;
       *reinterpret_cast<H4v*>(ks) = hi;
       *reinterpret_cast<H4v*>(ks + kKB * kKH) = lo;
     }
 #pragma unroll
-    for (int i = 0; i < kVPer; ++i) {
+    for (int i = 0; i < (kImg ? 0 : kVPer); ++i) {
       const int u = tid + i * nt, jq = u & 7, c4 = (u >> 3) & 31, bb = u >> 8;
       if (kVUnits % nt != 0 && u >= kVUnits) break;
-      const int slot = jq < 4 ? 8 * jq : 8 * (jq - 4) + 4;  // keys 4 jq .. + 3 in slot order
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
-        // dimension 4 c4 + d of the block: its 32 keys sit in 8 adjacent lanes
-        float mx = fmaxf(fmaxf(fabsf(vreg[i][0][d]), fabsf(vreg[i][1][d])),
-                         fmaxf(fabsf(vreg[i][2][d]), fabsf(vreg[i][3][d])));
-        const int se = ScaleExp(Max8Lanes(mx));
-        const float sv = Pow2(se);
-        if (jq == 0) vinv[bb][4 * c4 + d] = Pow2(-se);
-        _Float16* vt = kv + kBS * kKbH + bb * kVbH + (4 * c4 + d) * kVH + slot;
+        _Float16* vt = kv + kBS * kKbH + bb * kVbH + (4 * c4 + d) * kVH + VSlot(jq);
         H4v hi, lo;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) SplitHalf(vreg[i][r][d] * sv, hi, lo, r);
+        float inv;
+        SplitVUnit(F4v{vreg[i][0][d], vreg[i][1][d], vreg[i][2][d], vreg[i][3][d]}, &hi, &lo, &inv);
+        if (jq == 0) vinv[bb][4 * c4 + d] = inv;
         *reinterpret_cast<H4v*>(vt) = hi;
         *reinterpret_cast<H4v*>(vt + kHd * kVH) = lo;
       }
@@ -579,38 +689,58 @@ void Attention(const AttnArgs& a, hipStream_t s) {
     const int64_t n_keys_max = static_cast<int64_t>(a.pos0_host) + a.seq;
     RPG_CHECK(a.pos0_host >= 0 && n_keys_max <= a.max_seq, "attention past the cache capacity");
     const int64_t q_blocks = CeilDiv(a.seq, kQB);
+    AttnArgs b = a;
+    // the scratch holds the key blocks' images, then the partial states
+    const int64_t blocks = CeilDiv(n_keys_max, kKB), img_floats = a.n_kv * blocks * kImgFloats;
+    const bool img = q_blocks >= kImageQueryBlocks && a.part != nullptr && a.part_floats >= img_floats;
+    if (img) {
+      b.image = a.part;
+      b.image_blocks = blocks;
+      b.part = a.part + img_floats;
+      b.part_floats = a.part_floats - img_floats;
+      hipLaunchKernelGGL(KvImageKernel, dim3(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(blocks)), dim3(256),
+                         0, s, b, static_cast<int>(n_keys_max));
+      HIP_CHECK(hipGetLastError());
+    }
     const int splits =
-        PrefillSplits(a.n_kv * q_blocks, CeilDiv(n_keys_max, 2 * kKB), a.part != nullptr ? a.part_floats : 0,
+        PrefillSplits(a.n_kv * q_blocks, CeilDiv(n_keys_max, 2 * kKB), b.part != nullptr ? b.part_floats : 0,
                       static_cast<int64_t>(a.seq) * a.n_heads * (kHd + 2));
     const dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(q_blocks), static_cast<unsigned>(splits));
     // long segments at G <= 2: two query tiles per workgroup (half the
     // workgroups, each staged K/V block read by twice the queries)
     const bool wide = a.seq >= kWideQueries && CeilDiv(a.seq, 2 * kQB) * a.n_kv >= 256;
     const dim3 grid2(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(CeilDiv(a.seq, 2 * kQB)));
-    switch (a.n_heads / a.n_kv) {
-      case 1:
-        if (wide)
-          hipLaunchKernelGGL((PrefillKernel<1, 2>), grid2, dim3(256), 0, s, a);
-        else
-          hipLaunchKernelGGL((PrefillKernel<1, 1>), grid, dim3(128), 0, s, a);
-        break;
-      case 2:
-        if (wide)
-          hipLaunchKernelGGL((PrefillKernel<2, 2>), grid2, dim3(512), 0, s, a);
-        else
-          hipLaunchKernelGGL((PrefillKernel<2, 1>), grid, dim3(256), 0, s, a);
-        break;
-      case 3: hipLaunchKernelGGL((PrefillKernel<3, 1>), grid, dim3(384), 0, s, a); break;
-      case 4: hipLaunchKernelGGL((PrefillKernel<4, 1>), grid, dim3(512), 0, s, a); break;
-      case 5: hipLaunchKernelGGL((PrefillKernel<5, 1>), grid, dim3(640), 0, s, a); break;
-      case 6: hipLaunchKernelGGL((PrefillKernel<6, 1>), grid, dim3(768), 0, s, a); break;
-      case 7: hipLaunchKernelGGL((PrefillKernel<7, 1>), grid, dim3(896), 0, s, a); break;
-      default: hipLaunchKernelGGL((PrefillKernel<8, 1>), grid, dim3(1024), 0, s, a); break;
-    }
+    auto launch = [&](auto img_c) {
+      constexpr bool I = decltype(img_c)::value;
+      switch (a.n_heads / a.n_kv) {
+        case 1:
+          if (wide)
+            hipLaunchKernelGGL((PrefillKernel<1, 2, I>), grid2, dim3(256), 0, s, b);
+          else
+            hipLaunchKernelGGL((PrefillKernel<1, 1, I>), grid, dim3(128), 0, s, b);
+          break;
+        case 2:
+          if (wide)
+            hipLaunchKernelGGL((PrefillKernel<2, 2, I>), grid2, dim3(512), 0, s, b);
+          else
+            hipLaunchKernelGGL((PrefillKernel<2, 1, I>), grid, dim3(256), 0, s, b);
+          break;
+        case 3: hipLaunchKernelGGL((PrefillKernel<3, 1, I>), grid, dim3(384), 0, s, b); break;
+        case 4: hipLaunchKernelGGL((PrefillKernel<4, 1, I>), grid, dim3(512), 0, s, b); break;
+        case 5: hipLaunchKernelGGL((PrefillKernel<5, 1, I>), grid, dim3(640), 0, s, b); break;
+        case 6: hipLaunchKernelGGL((PrefillKernel<6, 1, I>), grid, dim3(768), 0, s, b); break;
+        case 7: hipLaunchKernelGGL((PrefillKernel<7, 1, I>), grid, dim3(896), 0, s, b); break;
+        default: hipLaunchKernelGGL((PrefillKernel<8, 1, I>), grid, dim3(1024), 0, s, b); break;
+      }
+    };
+    if (img)
+      launch(std::true_type{});
+    else
+      launch(std::false_type{});
     if (!wide && splits > 1) {
       HIP_CHECK(hipGetLastError());
       const int64_t rows = static_cast<int64_t>(a.seq) * a.n_heads;
-      hipLaunchKernelGGL(MergePrefillKernel, dim3(static_cast<unsigned>(CeilDiv(rows, 4))), dim3(256), 0, s, a, splits);
+      hipLaunchKernelGGL(MergePrefillKernel, dim3(static_cast<unsigned>(CeilDiv(rows, 4))), dim3(256), 0, s, b, splits);
     }
   }
   HIP_CHECK(hipGetLastError());

@@ -112,6 +112,9 @@ struct AttnArgs {
   // be null (no split)
   float* part = nullptr;
   int64_t part_floats = 0;
+  // (set by Attention: the key blocks' f16 images, in part)
+  float* image = nullptr;
+  int64_t image_blocks = 0;
 };
 int64_t AttnWorkFloats(int n_heads, int64_t max_seq);
 void Attention(const AttnArgs& a, hipStream_t s);
