@@ -612,14 +612,15 @@ int ChooseSplit(int64_t wgs, int nblk, int64_t cols, const SplitX& x, int64_t ta
 // The K parts (1 .. kTiledSplitMax) of `wgs` tiled workgroups of `nblk`
 // super-blocks on `cus` compute units (one tiled workgroup per unit): the
 // count whose rounds of workgroups take the least time, a workgroup costing
-// its super-blocks plus about 1.5 of pipeline fill and output. Every part
-// keeps at least 2.5 super-blocks on average, and at most `max_parts` partial
-// tiles are written.
+// its super-blocks plus about 1.5 of pipeline fill and output (0.8 and 2.5
+// measured the same). Every part keeps at least 1.67 super-blocks on average
+// (2.5 left the 1.7B shapes 2 - 4 % slower at 128 - 512 tokens, 1 no faster
+// than 1.67), and at most `max_parts` partial tiles are written.
 int TiledParts(int64_t wgs, int nblk, int64_t cus, int64_t max_parts) {
   int best = 1;
   double best_cost = 0.0;
   for (int c = 1; c <= kTiledSplitMax; ++c) {
-    if (c > 1 && (5 * c > 2 * nblk || c * wgs > max_parts)) break;
+    if (c > 1 && (10 * c > 6 * nblk || c * wgs > max_parts)) break;
     const double cost = static_cast<double>(CeilDiv(c * wgs, cus)) * (static_cast<double>(nblk) / c + 1.5);
     if (c == 1 || cost < 0.95 * best_cost) best = c, best_cost = cost;
   }
