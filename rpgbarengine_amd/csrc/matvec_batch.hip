@@ -735,7 +735,8 @@ int FewTokenLimit() {
 // QKV (15.7 M) 27 / 26, O (10.5 M) 18 / 23; 48 tokens, 1.7B Q8_0 gate+up
 // (25.2 M) 44 / 37, down (12.6 M) 31 / 32.
 bool FewTokensWin(int64_t weights, uint32_t type, int n) {
-  if (std::getenv("RPG_FEW_TOKENS") != nullptr) return true;  // (a sweep's limit alone decides)
+  static const bool sweep = EnvInt("RPG_FEW_TOKENS") > 0;
+  if (sweep) return true;  // (its limit alone decides)
   const bool q6 = type == kQ6_K, q8 = type == kQ8_0;
   const double w = static_cast<double>(weights) * 1e-6, groups = static_cast<double>(CeilDiv(n, 8));
   return 6.0 + (q6 ? 0.39 : q8 ? 0.25 : 0.19) * w * groups <= (q8 ? 25.0 : 22.0) + (q6 ? 0.4 : q8 ? 0.5 : 0.25) * w;
