@@ -455,11 +455,12 @@ void SwiGLURows(const float* g, const float* u, float* y, int64_t n, hipStream_t
 }
 
 namespace {
-// Floats of the split-K partials: tiled launches run at most kTiledPartTiles
-// partial tiles, whatever M.
-constexpr int64_t kTiledPartTiles = 512;
+// Floats of the split-K partials: tiled launches run at most this many partial
+// tiles, two rounds of 256 compute units; up to 64 tokens, whose row tiles are
+// few, one round (a session's first short segment allocates them).
+constexpr int64_t PartTiles(int M) { return M <= 64 ? 256 : 512; }
 int64_t PartFloats(int M, int n_max) {
-  return std::max<int64_t>(kTiledPartTiles * TiledTokens(M) * kTiledRows,
+  return std::max<int64_t>(PartTiles(M) * TiledTokens(M) * kTiledRows,
                            M < 96 ? static_cast<int64_t>(kGemmSplitMax) * M * n_max : 0);
 }
 }  // namespace
