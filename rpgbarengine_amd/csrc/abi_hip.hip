@@ -560,11 +560,8 @@ int32_t rpg_hip_attention(const float* q, const float* k, const float* v, int32_
     RPG_CHECK(seq > 0 && pos0 >= 0 && n_kv > 0 && n_heads > 0 && n_heads % n_kv == 0, "attention: bad shape");
     const int64_t n_pos = static_cast<int64_t>(pos0) + seq;
     const size_t qb = static_cast<size_t>(seq) * n_heads * 128 * 4, cb = static_cast<size_t>(n_kv) * n_pos * 128 * 4;
-    // the key blocks' images and the partial states of the most key ranges a
-    // launch may take
-    const int64_t part = n_kv * CeilDiv(n_pos, 32) * (2 * 32 * 128 + 160) +
-                         std::min<int64_t>(32, CeilDiv(n_pos, 64)) * seq * n_heads * 130;
-    DevBuf dq(qb), dk(cb), dv(cb), dout(qb), dpart(static_cast<size_t>(part) * 4);
+    const int64_t image = k::AttnImageFloats(seq, n_kv, n_pos);
+    DevBuf dq(qb), dk(cb), dv(cb), dout(qb), dimage(static_cast<size_t>(image) * 4);
     HIP_CHECK(hipMemcpy(dq.p, q, qb, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(dk.p, k, cb, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(dv.p, v, cb, hipMemcpyHostToDevice));
@@ -579,8 +576,8 @@ int32_t rpg_hip_attention(const float* q, const float* k, const float* v, int32_
     a.hd = 128;
     a.max_seq = n_pos;
     a.pos0_host = pos0;
-    a.part = dpart.as<float>();
-    a.part_floats = part;
+    a.image = image > 0 ? dimage.as<float>() : nullptr;
+    a.image_floats = image;
     RPG_CHECK(seq > 1, "attention: the segment kernel takes seq >= 2");
     k::Attention(a, nullptr);
     HIP_CHECK(hipMemcpy(out, dout.p, qb, hipMemcpyDeviceToHost));

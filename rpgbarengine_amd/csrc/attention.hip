@@ -13,14 +13,16 @@
 // RoPE and the cache write folded in, is in decode.hip.)
 //
 // Prefill (several queries): PrefillKernel, workgroup (kv head, 16 or 32
-// queries, and where these leave compute units idle one of several key
-// ranges, merged by MergePrefillKernel), two waves per query head of the group splitting the key blocks,
+// queries), two waves per query head of the group splitting the key blocks,
 // scores and P.V as f16 hi/lo products on the matrix cores (16x16x32), K/V
-// blocks of 32 positions staged once for the group, online softmax.
+// blocks of 32 positions staged once for the group, online softmax. (Key
+// ranges over several workgroups, merged by a second launch, were faster where
+// few queries stand behind a long history, but regroup a query's sums: a
+// sampled reply is then another one than the same seed gave before, wherever
+// a draw falls between the two roundings.)
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -37,7 +39,6 @@ namespace {
 constexpr int kChunk = 64;  // positions per decode split
 constexpr int kHd = 128;
 constexpr int kMaxGroup = 8;
-constexpr int kMaxPrefillSplits = 32;  // key ranges of a split prefill attention (at most a wave's lanes)
 
 __device__ __forceinline__ float WaveMax(float v) {
 #pragma unroll
@@ -248,13 +249,20 @@ __device__ __forceinline__ void SplitVUnit(F4v x, H4v* hi, H4v* lo, float* inv) 
 // Keys 4 jq .. + 3 of a block in V^T slot order.
 __device__ __forceinline__ int VSlot(int jq) { return jq < 4 ? 8 * jq : 8 * (jq - 4) + 4; }
 
-// The images of every key block of the segment's history: grid (kv head,
-// block), 256 threads. Keys past the last one repeat it.
-__global__ __launch_bounds__(256) void KvImageKernel(AttnArgs a, int n_keys) {
-  const int kh = blockIdx.x, blk = blockIdx.y, tid = threadIdx.x;
+// The images of the segment's key blocks: grid (image, kv head), 256 threads.
+// The first image_blocks images are those of all keys; then comes, for every
+// query block (of `queries` queries), its own last one, in which the last key
+// that its queries see is repeated: a V scale follows a block's largest value,
+// so that with keys of later queries in it the small values of others could
+// lose their last bits.
+__global__ __launch_bounds__(256) void KvImageKernel(AttnArgs a, int queries) {
+  const int kh = blockIdx.y, tid = threadIdx.x, tail = static_cast<int>(blockIdx.x) - static_cast<int>(a.image_blocks);
+  const int n_all = a.pos0_host + a.seq;
+  const int n_keys = tail < 0 ? n_all : min(a.pos0_host + (tail + 1) * queries, n_all);
+  const int blk = tail < 0 ? static_cast<int>(blockIdx.x) : (n_keys - 1) / kKB;
   const float* kb = a.kcache + static_cast<int64_t>(kh) * a.max_seq * kHd;
   const float* vb = a.vcache + static_cast<int64_t>(kh) * a.max_seq * kHd;
-  float* img = a.image + (static_cast<int64_t>(kh) * gridDim.y + blk) * kImgFloats;
+  float* img = a.image + (static_cast<int64_t>(kh) * gridDim.x + blockIdx.x) * kImgFloats;
   _Float16* ki = reinterpret_cast<_Float16*>(img);
   _Float16* vi = ki + kImgHalfs;
   float* inv = img + kImgHalfs;
@@ -295,11 +303,9 @@ __global__ __launch_bounds__(256) void KvImageKernel(AttnArgs a, int n_keys) {
 // G: query heads per KV head. Two waves per head split the key blocks (even
 // and odd) and merge their online-softmax states at the end; QT query tiles
 // of 16 share the workgroup's staged K/V blocks (long segments at G <= 2:
-// half the staging per query), so a workgroup has 2 G QT waves. With
-// gridDim.z = S > 1, workgroup z takes the z-th of S ranges of the block's
-// key steps and leaves its state to MergePrefillKernel (a.part: the output
-// sums [z][query][head][128], then (m, l) [z][query][head]). kImg: the blocks
-// are staged from their images (KvImageKernel) instead of from the cache.
+// half the staging per query), so a workgroup has 2 G QT waves. kImg: the
+// blocks are staged from their images (KvImageKernel) instead of from the
+// cache, to the same bits.
 template <int G, int QT, bool kImg>
 __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   constexpr int nt = 128 * G * QT;
@@ -336,20 +342,7 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   const float* kb = a.kcache + static_cast<int64_t>(kh) * a.max_seq * kHd;
   const float* vb = a.vcache + static_cast<int64_t>(kh) * a.max_seq * kHd;
   const int n_blocks = (n_keys + kKB - 1) / kKB;
-  const int n_steps_all = (n_blocks + kBS - 1) / kBS;
-  const int n_split = static_cast<int>(gridDim.z), z = static_cast<int>(blockIdx.z);
-  const int st0 = z * n_steps_all / n_split, n_steps = (z + 1) * n_steps_all / n_split;
-  float2* const part_ml =
-      reinterpret_cast<float2*>(a.part + static_cast<int64_t>(n_split) * a.seq * a.n_heads * kHd);
-  if (st0 == n_steps) {
-    // more ranges than steps: an empty state
-    for (int i = tid; i < kQB * QT * G; i += nt) {
-      const int t = t0b + i / G;
-      if (t < a.seq)
-        part_ml[(static_cast<int64_t>(z) * a.seq + t) * a.n_heads + kh * G + i % G] = float2{-__builtin_inff(), 0.0f};
-    }
-    return;
-  }
+  const int n_steps = (n_blocks + kBS - 1) / kBS;
   // step i stages blocks kBS i .. kBS i + kBS - 1: K as float4 units u = block
   // (u / 1024), key ((u / 32) % 32), column (u % 32) (32 lanes read one key
   // row and write it contiguously); V as units of 4 keys x
@@ -371,19 +364,23 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   constexpr int kSUnits = kBS * (kKB + kHd) / 4;
   static_assert(kSUnits <= nt, "a thread per four scales");
   F4v ireg[kImg ? kIPer : 1], sreg = F4v{0.f, 0.f, 0.f, 0.f};
-  const float* img = kImg ? a.image + static_cast<int64_t>(kh) * a.image_blocks * kImgFloats : nullptr;
+  const float* img =
+      kImg ? a.image + static_cast<int64_t>(kh) * (a.image_blocks + gridDim.y) * kImgFloats : nullptr;
+  auto image = [&](int blk) {
+    return img + static_cast<int64_t>(blk < n_blocks - 1 ? blk : static_cast<int>(a.image_blocks) + qb) * kImgFloats;
+  };
   auto load_step = [&](int st) {
     if constexpr (kImg) {
 #pragma unroll
       for (int i = 0; i < kIPer; ++i) {
         const int u = min(tid + i * nt, kIUnits - 1);
-        const float* p = img + static_cast<int64_t>(min(kBS * st + (u >> 11), n_blocks - 1)) * kImgFloats;
+        const float* p = image(kBS * st + (u >> 11));
         ireg[i] = *(const __attribute__((address_space(1))) F4v*)(p + 4 * (u & 2047));
       }
       if (tid < kSUnits) {
         const int bb = tid / (kSUnits / kBS), q = tid % (kSUnits / kBS);
         sreg = *(const __attribute__((address_space(1))) F4v*)(
-            img + static_cast<int64_t>(min(kBS * st + bb, n_blocks - 1)) * kImgFloats + kImgHalfs + 4 * q);
+            image(kBS * st + bb) + kImgHalfs + 4 * q);
       }
       return;
     }
@@ -403,7 +400,7 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
       }
     }
   };
-  load_step(st0);
+  load_step(0);
   // (after the first K/V loads, so that both round trips overlap)
   // this lane's query row c16 (clamped past the segment: computed, not
   // stored), dimensions 32 c + 8 kg .. + 7 of chunk c, split hi + lo
@@ -434,7 +431,7 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) SplitHalf(x[c][i] * sq, qh[c], ql[c], i);
   }
-  for (int st = st0; st < n_steps; ++st) {
+  for (int st = 0; st < n_steps; ++st) {
     __syncthreads();  // the previous step's LDS reads are done
     if constexpr (kImg) {
 #pragma unroll
@@ -576,11 +573,8 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   if (half == 0) {
     const float m1 = xm[lane * 2], l1 = xm[lane * 2 + 1];
     const float mn = fmaxf(m, m1);
-    // (a range of keys past this query has seen none: m = -inf, l = 0)
-    const bool none = mn == -__builtin_inff();
-    f0 = none ? 0.0f : ExpSoft(m - mn);
-    f1 = none ? 0.0f : ExpSoft(m1 - mn);
-    m = mn;
+    f0 = ExpSoft(m - mn);
+    f1 = ExpSoft(m1 - mn);
     l = __builtin_fmaf(l, f0, l1 * f1);
   }
   float* xo = kvf + QT * G * 64 * 2 + (qt * G + hg) * 64 * 16;  // [lane][4 tiles x 4 dimensions]
@@ -604,73 +598,18 @@ __global__ __launch_bounds__(128 * G * QT) void PrefillKernel(AttnArgs a) {
   if (half != 0) return;
   const int t = t0 + c16;
   if (t >= a.seq) return;
-  if (n_split > 1) {
-    const int64_t row = (static_cast<int64_t>(z) * a.seq + t) * a.n_heads + h;
-    float* po = a.part + row * kHd + 4 * kg;
-#pragma unroll
-    for (int ct = 0; ct < 8; ++ct) *reinterpret_cast<F4v*>(po + 16 * ct) = o[ct];
-    if (kg == 0) part_ml[row] = float2{m, l};
-    return;
-  }
   float* out = a.out + (static_cast<int64_t>(t) * a.n_heads + h) * kHd + 4 * kg;
 #pragma unroll
   for (int ct = 0; ct < 8; ++ct)
     *reinterpret_cast<float4*>(out + 16 * ct) = make_float4(o[ct][0] / l, o[ct][1] / l, o[ct][2] / l, o[ct][3] / l);
 }
 
-// The split prefill attention's output: one wave per (query, head) adds its
-// S states, each rescaled by exp(m_z - max m), and divides by the summed l;
-// lane d takes dimensions 2 d and 2 d + 1. A state that saw no key (l = 0) is
-// not read: its sums may be unwritten.
-__global__ __launch_bounds__(256) void MergePrefillKernel(AttnArgs a, int n_split) {
-  const int64_t rows = static_cast<int64_t>(a.seq) * a.n_heads;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= rows) return;
-  const float2* ml = reinterpret_cast<const float2*>(a.part + n_split * rows * kHd);
-  float m = -__builtin_inff(), l = 0.0f;
-  if (lane < n_split) {
-    const float2 v = ml[lane * rows + row];
-    m = v.x, l = v.y;
-  }
-  const float mx = WaveMax(m);  // (finite: every query sees key 0)
-  const float f = l > 0.0f ? ExpSoft(m - mx) : 0.0f;
-  const float total = WaveSum(l * f);
-  const float2* po = reinterpret_cast<const float2*>(a.part + row * kHd) + lane;
-  float ox = 0.0f, oy = 0.0f;
-  for (int z0 = 0; z0 < n_split; z0 += 4) {
-    float2 v[4];
-    float fz[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int z = z0 + i;
-      fz[i] = z < n_split ? __shfl(f, z, 64) : 0.0f;  // (uniform)
-      v[i] = float2{0.0f, 0.0f};
-      if (fz[i] != 0.0f) v[i] = po[z * rows * (kHd / 2)];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ox = __builtin_fmaf(v[i].x, fz[i], ox);
-      oy = __builtin_fmaf(v[i].y, fz[i], oy);
-    }
-  }
-  reinterpret_cast<float2*>(a.out + row * kHd)[lane] = float2{ox / total, oy / total};
-}
-
-// Key ranges of a prefill attention of `wgs` workgroups whose longest query
-// block walks `steps` steps of 64 keys: enough ranges for about two
-// workgroups per compute unit (their LDS lets two share one), at most one per
-// step and at most what the partials' buffer holds. Two ranges do not pay for
-// the merge (512 tokens of the 4B shape: 31 + 7.5 us against 37); from three
-// on they do: 203 queries behind 1500 keys (104 workgroups, 4 ranges) 106 ->
-// 60 + 6 us, 37 behind 611 (24 workgroups, 11 ranges) 45.6 -> 17.8 + 4.8 us.
-int PrefillSplits(int64_t wgs, int64_t steps, int64_t part_floats, int64_t row_floats) {
-  const int64_t room = part_floats / row_floats;
-  const int64_t s = std::min<int64_t>({kMaxPrefillSplits, 512 / std::max<int64_t>(wgs, 1), steps, room});
-  return s < 3 ? 1 : static_cast<int>(s);
-}
-
 }  // namespace
+
+int64_t AttnImageFloats(int seq, int n_kv, int64_t n_keys) {
+  const int64_t q_blocks = CeilDiv(seq, kQB);
+  return q_blocks < kImageQueryBlocks ? 0 : n_kv * (CeilDiv(n_keys, kKB) + q_blocks) * kImgFloats;
+}
 
 int64_t AttnWorkFloats(int n_heads, int64_t max_seq) {
   return static_cast<int64_t>(n_heads) * CeilDiv(max_seq, kChunk) * (2 + kHd);
@@ -688,40 +627,28 @@ void Attention(const AttnArgs& a, hipStream_t s) {
     RPG_CHECK(a.pos0_dev == nullptr, "prefill attention takes a host position");
     const int64_t n_keys_max = static_cast<int64_t>(a.pos0_host) + a.seq;
     RPG_CHECK(a.pos0_host >= 0 && n_keys_max <= a.max_seq, "attention past the cache capacity");
-    const int64_t q_blocks = CeilDiv(a.seq, kQB);
-    AttnArgs b = a;
-    // the scratch holds the key blocks' images, then the partial states
-    const int64_t blocks = CeilDiv(n_keys_max, kKB), img_floats = a.n_kv * blocks * kImgFloats;
-    const bool img = q_blocks >= kImageQueryBlocks && a.part != nullptr && a.part_floats >= img_floats;
-    if (img) {
-      b.image = a.part;
-      b.image_blocks = blocks;
-      b.part = a.part + img_floats;
-      b.part_floats = a.part_floats - img_floats;
-      hipLaunchKernelGGL(KvImageKernel, dim3(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(blocks)), dim3(256),
-                         0, s, b, static_cast<int>(n_keys_max));
-      HIP_CHECK(hipGetLastError());
-    }
-    const int splits =
-        PrefillSplits(a.n_kv * q_blocks, CeilDiv(n_keys_max, 2 * kKB), b.part != nullptr ? b.part_floats : 0,
-                      static_cast<int64_t>(a.seq) * a.n_heads * (kHd + 2));
-    const dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(q_blocks), static_cast<unsigned>(splits));
     // long segments at G <= 2: two query tiles per workgroup (half the
     // workgroups, each staged K/V block read by twice the queries)
-    const bool wide = a.seq >= kWideQueries && CeilDiv(a.seq, 2 * kQB) * a.n_kv >= 256;
-    const dim3 grid2(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(CeilDiv(a.seq, 2 * kQB)));
+    const bool wide =
+        a.n_heads <= 2 * a.n_kv && a.seq >= kWideQueries && CeilDiv(a.seq, 2 * kQB) * a.n_kv >= 256;
+    const int queries = wide ? 2 * kQB : kQB;
+    const int64_t q_blocks = CeilDiv(a.seq, queries);
+    const dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(q_blocks));
+    AttnArgs b = a;
+    b.image_blocks = CeilDiv(n_keys_max, kKB);
+    const int64_t image_floats = AttnImageFloats(a.seq, a.n_kv, n_keys_max);
     auto launch = [&](auto img_c) {
       constexpr bool I = decltype(img_c)::value;
       switch (a.n_heads / a.n_kv) {
         case 1:
-          if (wide)
-            hipLaunchKernelGGL((PrefillKernel<1, 2, I>), grid2, dim3(256), 0, s, b);
+          if (I && wide)
+            hipLaunchKernelGGL((PrefillKernel<1, I ? 2 : 1, I>), grid, dim3(256), 0, s, b);
           else
             hipLaunchKernelGGL((PrefillKernel<1, 1, I>), grid, dim3(128), 0, s, b);
           break;
         case 2:
-          if (wide)
-            hipLaunchKernelGGL((PrefillKernel<2, 2, I>), grid2, dim3(512), 0, s, b);
+          if (I && wide)
+            hipLaunchKernelGGL((PrefillKernel<2, I ? 2 : 1, I>), grid, dim3(512), 0, s, b);
           else
             hipLaunchKernelGGL((PrefillKernel<2, 1, I>), grid, dim3(256), 0, s, b);
           break;
@@ -733,14 +660,17 @@ void Attention(const AttnArgs& a, hipStream_t s) {
         default: hipLaunchKernelGGL((PrefillKernel<8, 1, I>), grid, dim3(1024), 0, s, b); break;
       }
     };
-    if (img)
-      launch(std::true_type{});
-    else
-      launch(std::false_type{});
-    if (!wide && splits > 1) {
+    if (image_floats > 0) {
+      RPG_CHECK(a.image != nullptr && a.image_floats >= image_floats,
+                "attention: %lld floats of images in a scratch of %lld", (long long)image_floats,
+                (long long)a.image_floats);
+      hipLaunchKernelGGL(KvImageKernel,
+                         dim3(static_cast<unsigned>(b.image_blocks + q_blocks), static_cast<unsigned>(a.n_kv)),
+                         dim3(256), 0, s, b, queries);
       HIP_CHECK(hipGetLastError());
-      const int64_t rows = static_cast<int64_t>(a.seq) * a.n_heads;
-      hipLaunchKernelGGL(MergePrefillKernel, dim3(static_cast<unsigned>(CeilDiv(rows, 4))), dim3(256), 0, s, b, splits);
+      launch(std::true_type{});
+    } else {
+      launch(std::false_type{});  // (short: never wide)
     }
   }
   HIP_CHECK(hipGetLastError());

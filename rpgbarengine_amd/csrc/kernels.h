@@ -107,15 +107,16 @@ struct AttnArgs {
   int64_t max_seq;
   const int32_t* pos0_dev;
   int32_t pos0_host;
-  // partial states of several queries' attention, for splitting their keys
-  // over workgroups where the queries alone leave compute units idle; it may
-  // be null (no split)
-  float* part = nullptr;
-  int64_t part_floats = 0;
-  // (set by Attention: the key blocks' f16 images, in part)
+  // scratch of several queries' attention: the f16 images of the key blocks
+  // (AttnImageFloats)
   float* image = nullptr;
-  int64_t image_blocks = 0;
+  int64_t image_floats = 0;
+  int64_t image_blocks = 0;  // (set by Attention)
 };
+// Floats of the images of n_keys keys for a segment of up to seq queries; 0
+// where it is too short to use them (each query block then converts the keys
+// that it reads, to the same bits).
+int64_t AttnImageFloats(int seq, int n_kv, int64_t n_keys);
 int64_t AttnWorkFloats(int n_heads, int64_t max_seq);
 void Attention(const AttnArgs& a, hipStream_t s);
 

@@ -263,7 +263,11 @@ void Session::EnsureScratch(int64_t tokens, int64_t logit_rows) {
   if (tokens >= 2) {  // GEMM operands of multi-token segments
     alloc(&gu_, 2 * static_cast<int64_t>(c.intermediate));
     const int kmax = std::max({c.hidden, c.q_dim(), c.intermediate});
-    const size_t split_bytes = k::SplitXBytes(static_cast<int>(tokens), kmax, SplitColumns(c));
+    // (or the attention's images of a full cache, whatever was prefilled so
+    // far: a conversation grown by short turns takes them too)
+    const size_t split_bytes =
+        std::max(k::SplitXBytes(static_cast<int>(tokens), kmax, SplitColumns(c)),
+                 sizeof(float) * static_cast<size_t>(k::AttnImageFloats(static_cast<int>(tokens), c.n_kv_heads, max_seq_)));
     DeviceAlloc(&split_, split_bytes);
     split_bytes_ = static_cast<int64_t>(split_bytes);
   }
@@ -327,8 +331,8 @@ void Session::ForwardSegment(const int32_t* ids_dev, int64_t n, int64_t pos0, co
     aa.pos0_dev = pos_dev;
     aa.pos0_host = static_cast<int32_t>(pos0);
     // (the GEMMs' operand buffer is idle between the QKV and O projections)
-    aa.part = static_cast<float*>(split_);
-    aa.part_floats = split_ ? split_bytes_ / 4 : 0;
+    aa.image = static_cast<float*>(split_);
+    aa.image_floats = split_ ? split_bytes_ / 4 : 0;
     k::Attention(aa, stream_);
   });
   if (logit_rows == 1 && m_.lm_head_tiled().w != nullptr) {

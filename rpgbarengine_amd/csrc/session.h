@@ -118,7 +118,7 @@ class Session {
   float* logits_ = nullptr;  // [logit rows][vocab]
   float* gu_ = nullptr;      // [2][tokens][intermediate]: gate and up outputs of the GEMM path
   void* split_ = nullptr;    // split input of the GEMM path (k::SplitXBytes); between projections, the
-                             // partial states of the segment's attention
+                             // images of the segment's attention
   int64_t split_bytes_ = 0;
   int64_t logit_rows_cap_ = 0;
   float* attn_work_ = nullptr;

@@ -516,15 +516,14 @@ def test_prefill_attention_matches_oracle(seq, n_heads, n_kv, pos0, qscale):
 
 
 @pytest.mark.parametrize("seq,n_heads,n_kv,pos0", [
-    (3, 32, 8, 3990),   # a few queries behind a long history: 32 ranges of two steps
-    (200, 4, 1, 0),     # short first query blocks: empty ranges
-    (40, 8, 2, 150),    # ranges of one step, the last partly visible
-    (203, 32, 8, 1500), # 4 ranges of unequal length
+    (3, 32, 8, 3990),   # a few queries behind a long history
+    (200, 4, 1, 0),     # one KV head
+    (40, 8, 2, 150),    # the last step partly visible
+    (203, 32, 8, 1500), # key blocks converted once
     (18, 5, 1, 700),    # G = 5
 ])
-def test_prefill_attention_key_ranges(seq, n_heads, n_kv, pos0):
-    """Segments whose keys are split over workgroups and merged, against the
-    oracle at the unsplit kernel's bound."""
+def test_prefill_attention_behind_history(seq, n_heads, n_kv, pos0):
+    """Segments behind a history, against the oracle at the kernel's bound."""
     rng = np.random.default_rng(seq + pos0)
     q = rng.standard_normal((seq, n_heads, 128)).astype(np.float32)
     k = rng.standard_normal((n_kv, pos0 + seq, 128)).astype(np.float32)
