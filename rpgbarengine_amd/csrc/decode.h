@@ -68,10 +68,6 @@ constexpr int kMaxBatchTokens = 64;
 // measured on the 1.7B / 4B projection shapes). RPG_FEW_TOKENS overrides it
 // for tuning sweeps (1 .. kMaxBatchTokens).
 int FewTokenLimit();
-// Whether a projection of `weights` weights (type: of its matrices, the first
-// one's where they differ) of a segment of n <= FewTokenLimit() tokens stays
-// on the few-token matvec rather than the tiled GEMM.
-bool FewTokensWin(int64_t weights, uint32_t type, int n);
 struct DecodeBatchArgs {
   DecodeJob job[3];
   int64_t ldy[3] = {0, 0, 0};

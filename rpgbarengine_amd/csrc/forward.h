@@ -64,19 +64,13 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
   // A few tokens (the decode step of a batch of sessions) run on the
   // multi-token matrix-core matvec over the tile-major copies, the RMSNorm
   // folded into its staging; returns false when a job has no such copy.
-  // Projections where the tiled GEMM is faster at this length leave it.
   auto batch = [&](const float* in, int K, const float* norm_w, bool pair,
                    std::initializer_list<std::pair<const k::MatRef*, k::GemmJob>> jobs) {
     if (N > k::FewTokenLimit()) return false;
-    int64_t weights = 0;
-    for (const auto& jb : jobs) {
-      if (jb.first == nullptr || jb.first->w == nullptr) return false;
-      weights += static_cast<int64_t>(jb.first->rows) * jb.first->cols * (pair ? 2 : 1);
-    }
-    if (!k::FewTokensWin(weights, jobs.begin()->first->type, N)) return false;
     k::DecodeBatchArgs a;
     a.n_jobs = 0;
     for (const auto& jb : jobs) {
+      if (jb.first == nullptr || jb.first->w == nullptr) return false;
       k::DecodeJob& J = a.job[a.n_jobs];
       J.w = jb.first->w;
       J.row_bytes = jb.first->row_bytes;

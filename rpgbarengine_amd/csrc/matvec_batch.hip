@@ -79,7 +79,11 @@ typedef float F4 __attribute__((ext_vector_type(4)));
 typedef float F2 __attribute__((ext_vector_type(2)));
 
 constexpr int kLdsBudget = 150 * 1024;  // staged tokens + per-group sums of one workgroup
-constexpr int kFewTokensDefault = 64;  // measured: the few-token launches beat the GEMMs on every 1.7B / 4B shape up to 64 tokens
+// Segments of up to 64 tokens take the few-token launches. A wide projection of
+// some 40 tokens is faster on the GEMM (4B gate+up of 37 tokens 53 us against
+// 35), whose hi + lo operands hold 22 bits below a token's largest input,
+// though, against 22 below its 32-group's here, and 30 of a Q8_0 launch.
+constexpr int kFewTokensDefault = 64;
 constexpr int kRecBytes = 96;       // digit rows of one token and group (three digits)
 constexpr int kRecBytes4 = 128;     // the same with four digits (Q8_0 launches)
 constexpr int kXgBytes = 16;        // (1/s, sum x, sum x of half 0, of half 1)
@@ -725,21 +729,6 @@ int FewTokenLimit() {
     return e >= 1 && e <= kMaxBatchTokens ? e : kFewTokensDefault;
   }();
   return limit;
-}
-
-// Per million weights, the matvec takes about 0.19 us a group of 8 tokens
-// (0.25 for Q8_0; 0.39 for a Q6_K matrix, whose wide inputs make groups of 4)
-// beside 6 us; the GEMM, its operand split included, 0.25 us (0.5, 0.4) up to
-// 64 tokens beside 22 us (25). Measured, matvec / GEMM, us: 37 tokens, 4B
-// gate+up (49.8 M weights) 53 / 35, down (24.9 M) Q4_K 33 / 32, Q6_K 55 / 39,
-// QKV (15.7 M) 27 / 26, O (10.5 M) 18 / 23; 48 tokens, 1.7B Q8_0 gate+up
-// (25.2 M) 44 / 37, down (12.6 M) 31 / 32.
-bool FewTokensWin(int64_t weights, uint32_t type, int n) {
-  static const bool sweep = EnvInt("RPG_FEW_TOKENS") > 0;
-  if (sweep) return true;  // (its limit alone decides)
-  const bool q6 = type == kQ6_K, q8 = type == kQ8_0;
-  const double w = static_cast<double>(weights) * 1e-6, groups = static_cast<double>(CeilDiv(n, 8));
-  return 6.0 + (q6 ? 0.39 : q8 ? 0.25 : 0.19) * w * groups <= (q8 ? 25.0 : 22.0) + (q6 ? 0.4 : q8 ? 0.5 : 0.25) * w;
 }
 
 namespace {

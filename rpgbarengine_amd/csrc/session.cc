@@ -351,18 +351,6 @@ void Session::ForwardSegment(const int32_t* ids_dev, int64_t n, int64_t pos0, co
     lm.job[0].y = logits_;
     NormFirst(&lm);
     k::DecodeMatvec(lm, stream_);
-  } else if (logit_rows >= 2 && k::QGemmSupports(m_.lm_head())) {
-    // every position's logits: the matrix-core GEMM, the RMSNorm folded into
-    // the operand split (the dequant matvec below reads the weights once per
-    // 8 rows: 300 rows of the 4B shape 38 times)
-    const int rows = static_cast<int>(logit_rows);
-    const k::SplitX sx = k::SplitXView(split_, rows, H, SplitColumns(c));
-    k::SplitRows(x_ + (n - logit_rows) * H, H, rows, H, m_.output_norm(), c.rms_eps, sx, stream_);
-    k::GemmJob job;
-    job.w = m_.lm_head();
-    job.y = logits_;
-    job.ldy = c.vocab;
-    k::QGemm(sx, &job, 1, stream_);
   } else if (logit_rows > 0) {
     const int64_t r0 = n - logit_rows;
     k::RmsNormRows(x_ + r0 * H, H, m_.output_norm(), H, static_cast<int>(logit_rows), c.rms_eps, h_, H, stream_);

@@ -12,6 +12,7 @@ import pytest
 
 import oracle
 import rpgbarengine_amd as eng
+from rpgbarengine_amd import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +41,27 @@ def test_prefill_attention_bits(seq, n_heads, n_kv, pos0, crc):
     if seq < 1000:
         assert np.abs(got - oracle.attention(q, k, v, pos0)).max() <= 2e-5 * np.abs(v).max()
     assert _crc(got) == crc
+
+
+# Two layers of the 1.7B width (a gate+up pair of 16.8 M weights), a segment
+# per entry: (tokens, logits of every position wanted, CRC of the logits)
+SHORT = {
+    "q4_k_m": [(20, 0, 1949256523), (41, 0, 3275326450), (64, 0, 432836158), (2, 0, 1009124003),
+               (8, 1, 490016019), (40, 1, 3505451445), (64, 1, 3998693554)],
+    "q8_0": [(20, 0, 2284655582), (41, 0, 1172620475), (64, 0, 4085952823), (2, 0, 3567769502),
+             (8, 1, 1359826666), (40, 1, 1070287797), (64, 1, 3021317139)],
+}
+
+
+@pytest.mark.parametrize("mix", sorted(SHORT))
+def test_short_segment_bits(gguf_factory, mix):
+    """Segments of up to 64 tokens stay on the few-token matvec, and the logits
+    of every position on fp32 inputs, whatever a wider launch would take."""
+    model = eng.Model(gguf_factory("tiny", mix, hidden=2048, n_heads=16, ffn=4096), max_pos=1024)
+    s = model.session(1024)
+    rng = np.random.default_rng(6)
+    got = []
+    for n, every, _ in SHORT[mix]:
+        ids = rng.integers(0, 1024, n, dtype=np.int32)
+        got.append(_crc(s.prefill(ids, all_logits=bool(every))))
+    assert got == [c for _, _, c in SHORT[mix]]
