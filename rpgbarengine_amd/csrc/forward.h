@@ -119,16 +119,15 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
     const k::SplitX sx = k::SplitXView(b.split, N, K, b.split_cols);
     k::SplitRowsAdd(const_cast<float*>(in), K, N, K, norm_w, c.rms_eps, sx, pend, stream);
     pend = k::SplitPending{};
-    // one launch per weight type (Q4_K and Q6_K share one); a second type runs
-    // on the side stream beside the first, each with half of the split-K
-    // partial buffer
+    // one launch per weight type; a second type runs on the side stream
+    // beside the first, each with half of the split-K partial buffer
     k::GemmJob grp[3][3];
     int gn[3] = {0, 0, 0}, n_grp = 0, ga[3][3];
     bool done[3] = {false, false, false};
     for (int i = 0; i < ng; ++i) {
       if (done[i]) continue;
       for (int j = i; j < ng; ++j) {
-        if (!done[j] && k::QGemmShares(g[j].w, g[i].w)) {
+        if (!done[j] && g[j].w.type == g[i].w.type) {
           ga[n_grp][gn[n_grp]] = at[j];
           grp[n_grp][gn[n_grp]++] = g[j];
           done[j] = true;
@@ -140,19 +139,14 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
     k::SplitPending* const defer[3] = {out ? left[0] : nullptr, out ? left[1] : nullptr, nullptr};
     if (n_grp == 2) {
       k::SplitX sa = sx, sb = sx;
-      sa.part_floats = sx.part_floats / 2;
-      sb.part_floats = sx.part_floats / 2;
-      sb.part = sx.part + sa.part_floats;
+      sa.part_floats = sb.part_floats = sx.part_floats / 2;
+      sa.part_cap = sb.part_cap = sx.part_cap / 2;
+      sb.part = sx.part + sa.part_cap;
       HIP_CHECK(hipEventRecord(b.ev_fork, stream));
       HIP_CHECK(hipStreamWaitEvent(b.side, b.ev_fork, 0));
-      // (each plans for the compute units of its share of the rows)
-      int64_t rows[2] = {0, 0};
-      for (int i = 0; i < 2; ++i)
-        for (int j = 0; j < gn[i]; ++j) rows[i] += grp[i][j].w.rows;
-      const int side_cus = std::max<int>(1, static_cast<int>(k::ComputeUnits() * rows[1] / (rows[0] + rows[1])));
-      k::QGemm(sb, grp[1], gn[1], b.side, defer[1], side_cus);
+      k::QGemm(sb, grp[1], gn[1], b.side, defer[1]);
       HIP_CHECK(hipEventRecord(b.ev_join, b.side));
-      k::QGemm(sa, grp[0], gn[0], stream, defer[0], std::max(1, k::ComputeUnits() - side_cus));
+      k::QGemm(sa, grp[0], gn[0], stream, defer[0]);
       HIP_CHECK(hipStreamWaitEvent(stream, b.ev_join, 0));
     } else if (n_grp == 1 && gn[0] == 1 && grp[0][0].y == x && grp[0][0].epi == k::kAdd) {
       k::QGemm(sx, grp[0], 1, stream, &pend);  // a K split's sums stay pending

@@ -38,8 +38,11 @@ struct SplitX {
   void* sum_hi = nullptr;  // f16 [M][K/32]: sum of each 32 inputs * s/32, split
   void* sum_lo = nullptr;
   float* inv_s = nullptr;  // [M] 1/s
-  float* part = nullptr;   // split-K partial products of QGemm
-  int64_t part_floats = 0;
+  // split-K partial products of QGemm: part_cap floats, of which the K-quants'
+  // splits plan with part_floats, a function of the segment alone (a product's
+  // order of sums follows its split)
+  float* part = nullptr;
+  int64_t part_floats = 0, part_cap = 0;
   int32_t M = 0, K = 0;
 };
 // Bytes of a SplitX for up to M x K whose QGemm launches produce at most
@@ -71,58 +74,79 @@ struct GemmJob {
   int64_t ldy = 0;
   Epilogue epi = kStore;
 };
-// Whether jobs of two types share a QGemm launch.
-bool QGemmShares(const MatRef& a, const MatRef& b);
 // True when W can run on QGemm (K-quants need K a multiple of 256).
 bool QGemmSupports(const MatRef& w);
-// cus: the compute units the launch may count on (0: all), where another
-// runs beside it.
-void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, SplitPending* defer = nullptr,
-           int cus = 0);
+// Jobs of one launch have one type.
+void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, SplitPending* defer = nullptr);
 // (defer: one entry per job; a K split's sums are left to the caller, to add
 // or store before y is read -- SplitRowsAdd, QkNormRopeCache, ApplyPending.
 // defer[j].part stays null when nothing is pending)
 // gate.y[t][r] = silu(gate row r . x_t) * (up row r . x_t) in one launch,
 // the same bits as two QGemm products and SwiGLURows -- except where a tiled
-// launch runs its last round's tiles in K parts: those rows' sums are the
-// parts' sums added, within the products' row bound. Gate and up of one type
-// and shape that the tiled launch takes; false (nothing launched) otherwise.
+// launch runs its last round's tiles in K parts (Q4_K: halves, where that round
+// is at most half full): those rows' sums are the parts' sums added, within
+// the products' row bound. Q4_K or Q8_0 gate and up of one shape; for Q4_K only
+// where QGemm would not split K. False (nothing launched) otherwise.
 bool QGemmSwiGLU(const SplitX& x, const GemmJob& gate, const GemmJob& up, hipStream_t s);
 
 // y[i] = silu(g[i]) * u[i] (reference src/kernels.h:82-92), n elements.
 void SwiGLURows(const float* g, const float* u, float* y, int64_t n, hipStream_t s);
 
-// Tiled GEMM (gemm_tiled.hip; Q4_K, Q6_K, Q8_0 with K a multiple of 256): 64 or
-// 128 tokens x 256 weight rows per workgroup. The K-quants' GEMM at every
-// segment length, and Q8_0's at those widths. Tiles of 64 tokens fill the
-// compute units with fewer K parts and pad less; from about 320 tokens on the
-// 128-token tiles' fewer LDS bytes per product win (a segment behind 600
-// tokens, ms, 64 / 128-token tiles: 4B Q4_K_M 65 tokens 7.4 / 8.7, 160 8.1 /
-// 10.2, 203 10.0 / 10.7, 300 11.8 / 12.0, 384 13.3 / 12.9, 512 16.2 / 15.5;
-// 1.7B Q4_K_M 65 4.7 / 5.9, 300 6.2 / 7.5, 512 8.7 / 8.8).
-constexpr int kTiledRows = 256;
-inline int TiledTokens(int M) { return M <= 320 ? 64 : 128; }
-
-// The types a tiled launch may hold side by side (any other launch: one type).
-inline bool TiledMixes(uint32_t type) { return type == kQ4_K || type == kQ6_K; }
+// Tiled Q4_K / Q6_K GEMM (gemm_tiled.hip): 128 tokens x 128 weight rows per
+// workgroup, each step's weights unpacked once into LDS. QGemm and QGemmSwiGLU
+// take it for segments of at least kTiledMinTokens tokens.
+// A kernel of 64 x 64 wave tiles with weights unpacked in registers, in the
+// form of gemm_q8.hip, ran these too and faster (4B 512 tokens 14.1 -> 12.7 ms,
+// 203 behind 1500 12.9 -> 9.5), closer to float64, but in another order of sums:
+// see QGemm's part_floats, and the replies that a seed gives.
+constexpr int kTiledTokens = 128;
+constexpr int kTiledRows = 128;
+constexpr int kTiledMinTokens = 96;
 
 struct TiledArgs {
   SplitX x;
   GemmJob job[3];
+  int32_t tiles[3];  // 128-row tiles per job (pair: 64-row tiles of gate and up)
+  int32_t n_jobs;
+  int32_t tiles_m;   // 128-token tiles; workgroup i takes token tile i % tiles_m
+  int32_t ksplit;    // blockIdx.y takes super-blocks [y * n / ksplit, (y + 1) * n / ksplit)
+  int64_t part_ld;   // partials: x.part[(z * M + token) * part_ld + pcol[job] + row]
+  int32_t pcol[3];
+  int32_t pair;      // job 0 gate, job 1 up: y = silu(gate.x) * (up.x), no K split
+  // pair only, 0 = none: workgroups from tail_wg on take the tiles from
+  // tail_wg on in halves (the two super-block halves of each, raw sums to
+  // x.part, kTiledTailFloats per half), finished by a second launch
+  int32_t tail_wg = 0;
+};
+constexpr int kTiledTailFloats = kTiledTokens * kTiledRows;
+void LaunchTiled(const TiledArgs& a, hipStream_t s);
+
+// Tiled Q8_0 GEMM (gemm_q8.hip; K a multiple of 256): 64 or 128 tokens x 256
+// weight rows per workgroup. Tiles of 64 tokens fill the compute units with
+// fewer K parts and pad less; from about 320 tokens on the 128-token tiles'
+// fewer LDS bytes per product win (measured on the kernel's Q4_K form, a
+// segment behind 600 tokens, ms, 64 / 128-token tiles: 1.7B 65 tokens 4.7 / 5.9,
+// 300 6.2 / 7.5, 512 8.7 / 8.8).
+constexpr int kQ8Rows = 256;
+inline int Q8TileTokens(int M) { return M <= 320 ? 64 : 128; }
+
+struct Q8TiledArgs {
+  SplitX x;
+  GemmJob job[3];
   int32_t tiles[3];  // 256-row tiles per job (pair: 128-row tiles of gate and up)
   int32_t n_jobs;
-  int32_t tokens;    // TiledTokens(x.M)
+  int32_t tokens;    // Q8TileTokens(x.M)
   int32_t tiles_m;   // token tiles; workgroup i takes token tile i % tiles_m
   int32_t ksplit;    // blockIdx.y takes super-blocks [y * n / ksplit, (y + 1) * n / ksplit)
   int64_t part_ld;   // partials: x.part[(z * M + token) * part_ld + pcol[job] + row]
   int32_t pcol[3];
   int32_t pair;      // job 0 gate, job 1 up: y = silu(gate.x) * (up.x), no K split
   // pair only, tail_split > 1: the tiles from tail_wg on run as tail_split K
-  // parts each (raw sums to x.part, tokens x kTiledRows floats per part),
-  // finished by a second launch
+  // parts each (raw sums to x.part, tokens x kQ8Rows floats per part), finished
+  // by a second launch
   int32_t tail_wg = 0, tail_split = 1;
 };
-void LaunchTiled(const TiledArgs& a, hipStream_t s);
+void LaunchQ8Tiled(const Q8TiledArgs& a, hipStream_t s);
 
 }  // namespace k
 }  // namespace rpg

@@ -65,3 +65,61 @@ def test_short_segment_bits(gguf_factory, mix):
         ids = rng.integers(0, 1024, n, dtype=np.int32)
         got.append(_crc(s.prefill(ids, all_logits=bool(every))))
     assert got == [c for _, _, c in SHORT[mix]]
+
+
+# 24 tokens on the few-token matvec, 65 and 95 on the 32-token kernels, the rest
+# on the tiled one: K splits of one to four parts
+@pytest.mark.parametrize("qtype,k,rows,m,crc", [
+    (synth.Q4_K, 2560, 300, 24, 263964610), (synth.Q4_K, 2560, 1000, 65, 514150326),
+    (synth.Q4_K, 2560, 1000, 95, 1752270011), (synth.Q4_K, 2560, 1000, 96, 592997306),
+    (synth.Q4_K, 9728, 513, 130, 1119775581), (synth.Q4_K, 2560, 6144, 512, 1719389901),
+    (synth.Q4_K, 256, 1, 100, 4253233896), (synth.Q4_K, 4096, 2560, 333, 3376873728),
+    (synth.Q4_K, 2304, 640, 900, 2955258594), (synth.Q6_K, 2560, 300, 24, 2335545069),
+    (synth.Q6_K, 2560, 1000, 65, 2692310153), (synth.Q6_K, 2560, 1000, 95, 795841049),
+    (synth.Q6_K, 2560, 1000, 96, 2543986180), (synth.Q6_K, 9728, 513, 130, 3445473103),
+    (synth.Q6_K, 2560, 6144, 512, 1992489358), (synth.Q6_K, 256, 1, 100, 605201952),
+    (synth.Q6_K, 4096, 2560, 333, 4250083847), (synth.Q6_K, 2304, 640, 900, 3129518966),
+])
+def test_kquant_product_bits(qtype, k, rows, m, crc):
+    """Inputs with a heavy tail (cubed normals)."""
+    raw = synth.quantize(qtype, synth.gaussian(71, k + rows + qtype, rows * k, 0.02).reshape(rows, k))
+    X = synth.gaussian(72, k + m, m * k, 1.0).reshape(m, k) ** 3
+    assert _crc(eng.matmul(qtype, raw, rows, k, X)) == crc
+
+
+@pytest.mark.parametrize("k,rows,m,fused,crc", [
+    (2560, 1000, 70, True, 1717677690), (2560, 2560, 101, False, 451792006), (1024, 2820, 900, True, 3251317571),
+    (2560, 9728, 512, True, 3292148604), (512, 2560, 900, True, 2681902950),
+])
+def test_q4k_gate_up_bits(k, rows, m, fused, crc):
+    g = synth.quantize(synth.Q4_K, synth.gaussian(73, k + rows, rows * k, 0.02).reshape(rows, k))
+    u = synth.quantize(synth.Q4_K, synth.gaussian(74, k + rows, rows * k, 0.02).reshape(rows, k))
+    X = synth.gaussian(75, k + m, m * k, 1.0).reshape(m, k)
+    y, one_launch = eng.matmul_swiglu(synth.Q4_K, g, u, rows, k, X)
+    assert one_launch == fused and _crc(y) == crc
+
+
+def test_conversation_bits(gguf_factory):
+    """A Q4_K_M conversation of growing and shrinking segments, a sampled
+    reply, scores, and two batches of sampled replies."""
+    model = eng.Model(gguf_factory("mid", "q4_k_m"), max_pos=2048)
+    rng = np.random.default_rng(5)
+
+    def ids(n):
+        return rng.integers(0, 32000, n, dtype=np.int32)
+
+    s = model.session(2048)
+    turns = [(700, 2611664729), (24, 3362935199), (130, 3519248235), (1, 1733760205), (64, 2136527876),
+             (65, 3586634463), (300, 3345292912), (2, 1123258492)]
+    assert [(n, _crc(s.prefill(ids(n)))) for n, _ in turns] == turns
+    assert _crc(s.generate(24, 0.2, 0, 0.95, 77)) == 3017764523
+    s = model.session(1024)
+    s.prefill(ids(50))
+    scores = [(8, 2850593359), (40, 1962683207), (200, 501750474)]
+    assert [(n, _crc(s.prefill(ids(n), all_logits=True))) for n, _ in scores] == scores
+    for n, reply, after in [(3, 3979195660, 1440404889), (8, 1401735295, 1483802196)]:
+        sessions = [model.session(512) for _ in range(n)]
+        for x in sessions:
+            x.prefill(ids(100 + n))
+        got, _ = eng.generate_batch(sessions, 16, 0.2, 0, 0.95, [9 + i for i in range(n)])
+        assert (_crc(got), _crc(np.stack([x.prefill(ids(3)) for x in sessions]))) == (reply, after)

@@ -137,12 +137,13 @@ def test_tiled_gemm_ragged_shapes(qtype, k, rows, m):
     assert np.all(Y[m - 1] == 0.0)
 
 
-# The tiled kernel's Q8_0 form and its K parts: token and row tiles partly
-# empty, one row, part ranges of unequal length (38 super-blocks in 8).
+# The tiled Q8_0 kernel and its K parts: token and row tiles partly empty, one
+# row, part ranges of unequal length (38 super-blocks in 8). The K-quants beside
+# it in theirs.
 @pytest.mark.parametrize("qtype,k,rows,m", [(synth.Q8_0, 2560, 300, 130), (synth.Q8_0, 256, 1, 100),
                                             (synth.Q8_0, 9728, 257, 129), (synth.Q6_K, 9728, 257, 129),
                                             (synth.Q4_K, 9728, 513, 97)])
-def test_tiled_gemm_256_rows(qtype, k, rows, m):
+def test_tiled_gemm_parts(qtype, k, rows, m):
     w32 = synth.gaussian(41, k + rows + qtype, rows * k, 0.02).reshape(rows, k)
     raw = synth.quantize(qtype, w32)
     wdq = oracle.dequant(qtype, raw.reshape(-1), rows * k).reshape(rows, k)
@@ -154,14 +155,15 @@ def test_tiled_gemm_256_rows(qtype, k, rows, m):
     assert np.all(Y[m - 1] == 0.0)
 
 
-@pytest.mark.parametrize("qtype", TYPES)
-def test_tiled_gemm_common_error(qtype):
-    """The matrix core rounds its sums down; the tiled kernel's alternating
-    signs cancel that. Inputs with a heavy tail (cubed normals): the mean
-    error over 65536 outputs, each with an error of about 2e-7 of the outputs'
-    root mean square shared by up to 256 tokens of a row, stays below
-    6e-8 (without the signs it measured 1e-7 and more on long chains)."""
-    k, rows, m = 2048, 256, 256
+@pytest.mark.parametrize("m", [256, 512])
+def test_tiled_gemm_common_error(m):
+    """The matrix core rounds its sums down; the tiled Q8_0 kernel's alternating
+    signs cancel that, with tiles of 64 and of 128 tokens. Inputs with a heavy
+    tail (cubed normals): the mean error over all outputs, each with an error
+    of about 2e-7 of the outputs' root mean square shared by up to m tokens of a
+    row, stays below 6e-8 (without the signs it measured 1e-7 and more on long
+    chains)."""
+    qtype, k, rows = synth.Q8_0, 2048, 256
     w32 = synth.gaussian(51, k + qtype, rows * k, 0.02).reshape(rows, k)
     raw = synth.quantize(qtype, w32)
     wdq = oracle.dequant(qtype, raw.reshape(-1), rows * k).reshape(rows, k).astype(np.float64)
@@ -173,8 +175,8 @@ def test_tiled_gemm_common_error(qtype):
 
 # A fused gate/up/SwiGLU launch whose tiles run in K parts: every tile (one
 # token tile, a partial row tile), and the tiles past a full round of 256
-# compute units (23 x 12 = 276) -- Q4_K and Q8_0.
-@pytest.mark.parametrize("qtype,rows,k,m", [(synth.Q4_K, 1000, 2560, 101), (synth.Q8_0, 1000, 2560, 101),
+# compute units -- Q8_0 (23 x 12 tiles), Q4_K (45 x 12, halves).
+@pytest.mark.parametrize("qtype,rows,k,m", [(synth.Q8_0, 1000, 2560, 101), (synth.Q8_0, 2820, 2560, 1413),
                                             (synth.Q4_K, 2820, 2560, 1413)])
 def test_gate_up_swiglu_tail_parts(qtype, rows, k, m):
     g = synth.quantize(qtype, synth.gaussian(61, rows + k, rows * k, 0.02).reshape(rows, k))
