@@ -585,6 +585,21 @@ int32_t rpg_hip_attention(const float* q, const float* k, const float* v, int32_
   }, -1);
 }
 
+int32_t rpg_hip_split_layout(int32_t tokens, int32_t k, int32_t columns, int64_t* out) {
+  return Guard([&]() -> int32_t {
+    RPG_CHECK(tokens > 0 && k > 0 && columns > 0, "split_layout: empty shape");
+    // (256: an address to tell the parts apart by, nothing is read there)
+    const k::SplitX x = k::SplitXView(reinterpret_cast<void*>(256), tokens, k, columns);
+    const auto at = [](const void* p) { return static_cast<int64_t>(reinterpret_cast<uintptr_t>(p)) - 256; };
+    out[0] = at(x.hi);
+    out[1] = at(x.inv_s + tokens);
+    out[2] = at(x.part);
+    out[3] = at(x.part + x.part_cap);
+    out[4] = static_cast<int64_t>(k::SplitXBytes(tokens, k, columns));
+    return 0;
+  }, -1);
+}
+
 int32_t rpg_hip_expf(const float* x, int64_t n, float* out) {
   return Guard([&]() -> int32_t {
     RequireGpu();

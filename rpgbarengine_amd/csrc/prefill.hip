@@ -1009,14 +1009,17 @@ size_t SplitXBytes(int M, int K, int n_max) {
 SplitX SplitXView(void* base, int M, int K, int n_max) {
   const size_t big = static_cast<size_t>(M) * K * 2, small = static_cast<size_t>(M) * (K / 32) * 2;
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-  uint8_t* p = static_cast<uint8_t*>(base);
+  // The partial sums first, at an offset that does not depend on K: one
+  // projection's stay there until the next one's operands are split (of another
+  // width), each token's workgroup adding its own while others write operands.
+  uint8_t* p = static_cast<uint8_t*>(base) + up(static_cast<size_t>(PartCap(M, n_max)) * 4);
   SplitX s;
+  s.part = static_cast<float*>(base);
   s.hi = p;
   s.lo = p + up(big);
   s.sum_hi = p + 2 * up(big);
   s.sum_lo = p + 2 * up(big) + up(small);
   s.inv_s = reinterpret_cast<float*>(p + 2 * up(big) + 2 * up(small));
-  s.part = reinterpret_cast<float*>(p + 2 * up(big) + 2 * up(small) + up(static_cast<size_t>(M) * 4));
   s.part_floats = PartFloats(M, n_max);
   s.part_cap = PartCap(M, n_max);
   s.M = M;
@@ -1032,6 +1035,12 @@ void SplitRowsAdd(float* X, int64_t ldx, int M, int K, const float* norm_w, floa
   RPG_CHECK(pend.part == nullptr || (pend.M == M && (pend.part_ld + pend.pcol) % 4 == 0 && pend.pcol % 4 == 0 &&
                                       pend.ksplit >= 1 && pend.ksplit <= kSplitPendMax),
             "split rows: pending sums do not match the rows");
+  if (pend.part != nullptr) {
+    const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+    RPG_CHECK(at(pend.part + static_cast<int64_t>(pend.ksplit) * M * pend.part_ld) <= at(out.hi) ||
+                  at(out.inv_s + M) <= at(pend.part),
+              "split rows: pending sums among the operands");
+  }
   SplitX o = out;
   o.M = M;
   const dim3 grid(static_cast<unsigned>(M));
