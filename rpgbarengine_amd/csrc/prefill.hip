@@ -1091,10 +1091,16 @@ void SplitRows(const float* X, int64_t ldx, int M, int K, const float* norm_w, f
 }
 
 namespace {
-// Whether the tiled Q8_0 kernel takes the matrix (its lane offsets are 32-bit).
-bool Q8TiledTakes(const MatRef& w) {
-  return w.type == kQ8_0 && w.cols % 256 == 0 && w.row_bytes * w.rows < 0xFFFF0000LL;
+// Whether a tiled kernel reaches every byte of the matrix and of the operands of
+// M tokens (past the last ones to a whole tile): its offsets are 32-bit, those of
+// a token row and of a step added up. The other kernels address with 64 bits.
+bool TiledReaches(const MatRef& w, int M) {
+  return w.row_bytes * w.rows < 0xFFFF0000LL && (static_cast<int64_t>(M) + 128) * w.cols * 2 < 0x7FFF0000LL;
 }
+bool KTiledTakes(const MatRef& w, int M) {
+  return (w.type == kQ4_K || w.type == kQ6_K) && M >= kTiledMinTokens && TiledReaches(w, M);
+}
+bool Q8TiledTakes(const MatRef& w, int M) { return w.type == kQ8_0 && w.cols % 256 == 0 && TiledReaches(w, M); }
 }  // namespace
 
 bool QGemmSupports(const MatRef& w) {
@@ -1195,13 +1201,16 @@ void QGemm(const SplitX& x, const GemmJob* jobs, int n_jobs, hipStream_t s, Spli
   }
   int S = 1;
   const bool q6 = jobs[0].w.type == kQ6_K, kq = q6 || jobs[0].w.type == kQ4_K;
-  bool q8_tiled = true;
-  for (int j = 0; j < n_jobs; ++j) q8_tiled = q8_tiled && Q8TiledTakes(jobs[j].w);
+  bool k_tiled = true, q8_tiled = true;
+  for (int j = 0; j < n_jobs; ++j) {
+    k_tiled = k_tiled && KTiledTakes(jobs[j].w, x.M);
+    q8_tiled = q8_tiled && Q8TiledTakes(jobs[j].w, x.M);
+  }
   // Q4_K / Q6_K launches of long segments take the tiled kernel. (Its K
   // split fills at most one round of compute units, so the q,k launch -- 160
   // workgroups at 512 tokens -- leaves room for the v launch beside it on
   // the side stream.)
-  if (kq && x.M >= kTiledMinTokens) {
+  if (k_tiled) {
     TiledArgs t;
     t.x = x;
     t.pair = 0;
@@ -1316,7 +1325,7 @@ bool QGemmSwiGLU(const SplitX& x, const GemmJob& gate, const GemmJob& up, hipStr
       gate.w.row_bytes != up.w.row_bytes || x.K % 256 != 0)
     return false;
   const int64_t cus = ComputeUnits();
-  if (Q8TiledTakes(gate.w)) {
+  if (Q8TiledTakes(gate.w, x.M)) {
     Q8TiledArgs t;
     t.x = x;
     t.pair = 1;
@@ -1339,7 +1348,7 @@ bool QGemmSwiGLU(const SplitX& x, const GemmJob& gate, const GemmJob& up, hipStr
     return true;
   }
   if (gate.w.type != kQ4_K) return false;
-  if (x.M >= kTiledMinTokens) {
+  if (KTiledTakes(gate.w, x.M)) {
     // the tiled launch; fused only where the unfused one would not split
     const int64_t mt = CeilDiv(x.M, kTiledTokens);
     if (TiledSplit(2 * CeilDiv(gate.w.rows, kTiledRows) * mt, x.K / 256, 2 * static_cast<int64_t>(gate.w.rows), x) >

@@ -582,3 +582,37 @@ def test_prefill_attention_mixed_magnitudes():
     err = np.abs(got.astype(np.float64) - want).max(axis=(0, 1))
     vmax = np.abs(v).max(axis=(0, 1))
     assert np.all(err <= 2e-5 * vmax)
+
+
+# Past the 32-bit offsets of the tiled kernels (4 GiB of token operands, of
+# weights) the products run on the kernels that address with 64 bits.
+@pytest.mark.parametrize("qtype", [synth.Q8_0, synth.Q4_K])
+def test_matmul_operands_past_4_gib(qtype):
+    """8.4 M tokens of 256 inputs, all zero but some at both ends, around the
+    8388608th (4 GiB of f16) and between: those at the row bound, the rest 0."""
+    k, m = 256, 8_400_000
+    raw = synth.quantize(qtype, synth.gaussian(81, qtype, k, 0.02).reshape(1, k))
+    wdq = oracle.dequant(qtype, raw.reshape(-1), k).reshape(1, k)
+    rows = np.unique(np.concatenate([np.arange(70), np.arange(8388608 - 70, 8388608 + 70), np.arange(m - 70, m),
+                                     np.arange(1, m, 99991)]))
+    X = np.zeros((m, k), np.float32)
+    X[rows] = synth.gaussian(82, 0, rows.size * k, 1.0).reshape(-1, k)
+    Y = eng.matmul(qtype, raw, 1, k, X)
+    assert rel_row_error(Y[rows], X[rows], wdq) <= 1e-6
+    Y[rows] = 0.0
+    assert not Y.any()
+
+
+def test_matmul_weights_past_4_gib():
+    """A Q4_K matrix of 4.3 GB, 1024 rows over and over: each repeat gives the
+    same bits, at the row bound."""
+    k, m, base = 40960, 96, 1024
+    raw = synth.quantize(synth.Q4_K, synth.gaussian(83, 0, base * k, 0.02).reshape(base, k)).reshape(base, -1)
+    times = (1 << 32) // raw.size + 2
+    rows = times * base
+    X = synth.gaussian(84, 0, m * k, 1.0).reshape(m, k)
+    Y = eng.matmul(synth.Q4_K, np.tile(raw, (times, 1)), rows, k, X)
+    Y = Y.reshape(m, times, base)
+    assert all(np.array_equal(Y[:, t], Y[:, 0]) for t in range(1, times))
+    wdq = oracle.dequant(synth.Q4_K, raw.reshape(-1), base * k).reshape(base, k)
+    assert rel_row_error(Y[:, 0], X, wdq) <= 1e-6
