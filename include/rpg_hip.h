@@ -204,10 +204,11 @@ RPG_HIP_API int32_t rpg_hip_attention(const float* q, const float* k, const floa
                                       int32_t n_kv, int32_t pos0, float* out);
 
 /* Where the GEMM operands of a segment of `tokens` x k inputs and the partial
- * sums of its products (columns: of the widest launch) lie in their buffer:
- * out = {operands' begin, end, partials' begin, end, buffer size}, bytes. Host
+ * sums of its products (columns: of the widest launch; q8: Q8_0 weights among them) lie in their
+ * buffer: out = {operands' begin, end, partials' begin, end, buffer size}, bytes. Host
  * only. */
-RPG_HIP_API int32_t rpg_hip_split_layout(int32_t tokens, int32_t k, int32_t columns, int64_t* out);
+RPG_HIP_API int32_t rpg_hip_split_layout(int32_t tokens, int32_t k, int32_t columns, int32_t q8,
+                                         int64_t* out);
 
 /* glibc-exact expf on the GPU over n inputs (parity probe). */
 RPG_HIP_API int32_t rpg_hip_expf(const float* x, int64_t n, float* out);

@@ -73,7 +73,7 @@ _SIG = {
     "rpg_hip_sampler_tie_orders": ([], _I64),
     "rpg_hip_sample_noalloc": ([_P, _I32, _F, _I32, _F, _U64, _I64, _P, _P, _P], _I32),
     "rpg_hip_attention": ([_P, _P, _P, _I32, _I32, _I32, _I32, _P], _I32),
-    "rpg_hip_split_layout": ([_I32, _I32, _I32, _P], _I32),
+    "rpg_hip_split_layout": ([_I32, _I32, _I32, _I32, _P], _I32),
     "rpg_hip_expf": ([_P, _I64, _P], _I32),
     "rpg_hip_bench_matmul": ([_U32, _P, _I64, _I64, _P, _I32, _I32, _I32, _P], _I32),
 }
@@ -206,11 +206,11 @@ def sampler_tie_orders() -> int:
     return int(lib().rpg_hip_sampler_tie_orders())
 
 
-def split_layout(tokens: int, k: int, columns: int) -> np.ndarray:
+def split_layout(tokens: int, k: int, columns: int, q8: bool) -> np.ndarray:
     """(operands' begin, end, partials' begin, end, size) of a segment's GEMM
     buffer, in bytes."""
     out = np.zeros(5, dtype=np.int64)
-    _ok(lib().rpg_hip_split_layout(tokens, k, columns, _p(out)))
+    _ok(lib().rpg_hip_split_layout(tokens, k, columns, int(q8), _p(out)))
     return out
 
 

@@ -107,7 +107,7 @@ k::MatRef HostMat(uint32_t type, const uint8_t* w_dev, int64_t rows, int64_t col
 // Y = X . W^T the way the engine runs a projection of n tokens: up to
 // FewTokenLimit() through the decode matvecs on the tile-major copy when
 // there is one, more through the matrix-core GEMM when the weight type has
-// one (split buffer: k::SplitXBytes(n, cols, rows) bytes).
+// one (split buffer: k::SplitXBytes(n, cols, rows, Q8_0 or not) bytes).
 void Project(const k::MatRef& m, const float* X, int n, float* Y, void* split, hipStream_t s,
              const uint8_t* tiled = nullptr) {
   if (n == 1 && tiled != nullptr) {  // the decode step's path: the tile-major copy
@@ -136,7 +136,7 @@ void Project(const k::MatRef& m, const float* X, int n, float* Y, void* split, h
     a.ldy[0] = m.rows;
     RPG_CHECK(k::DecodeMatvecBatch(a, s), "matmul: the batch matvec refused %d tokens", n);
   } else if (n >= 2 && k::QGemmSupports(m)) {
-    const k::SplitX sx = k::SplitXView(split, n, m.cols, static_cast<int>(m.rows));
+    const k::SplitX sx = k::SplitXView(split, n, m.cols, static_cast<int>(m.rows), m.type == kQ8_0);
     k::SplitRows(X, m.cols, n, m.cols, nullptr, 0.0f, sx, s);
     k::GemmJob job;
     job.w = m;
@@ -439,7 +439,7 @@ int32_t rpg_hip_matmul(uint32_t type, const uint8_t* w, int64_t rows, int64_t co
     HIP_CHECK(hipMemcpy(dw.p, w, wb, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(dx.p, X, static_cast<size_t>(n * cols) * 4, hipMemcpyHostToDevice));
     const k::MatRef m = HostMat(type, dw.as<uint8_t>(), rows, cols);
-    DevBuf split(k::SplitXBytes(static_cast<int>(n), static_cast<int>(cols), static_cast<int>(rows)));
+    DevBuf split(k::SplitXBytes(static_cast<int>(n), static_cast<int>(cols), static_cast<int>(rows), type == kQ8_0));
     const bool tile = n == 1 ? k::DecodeTileable(m) : n <= k::FewTokenLimit() && k::BatchTileable(m);
     DevBuf tiled(tile ? static_cast<size_t>(k::TileMajorBytes(m, false)) : 16);
     if (tile) k::TileMajor(m, nullptr, tiled.as<uint8_t>(), nullptr);
@@ -504,8 +504,10 @@ int32_t rpg_hip_matmul_swiglu(uint32_t type, const uint8_t* gate, const uint8_t*
     HIP_CHECK(hipMemcpy(dg.p, gate, wb, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(du.p, up, wb, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(dx.p, X, static_cast<size_t>(n * cols) * 4, hipMemcpyHostToDevice));
-    DevBuf split(k::SplitXBytes(static_cast<int>(n), static_cast<int>(cols), static_cast<int>(2 * rows)));
-    const k::SplitX sx = k::SplitXView(split.p, static_cast<int>(n), static_cast<int>(cols), static_cast<int>(2 * rows));
+    DevBuf split(k::SplitXBytes(static_cast<int>(n), static_cast<int>(cols), static_cast<int>(2 * rows),
+                                type == kQ8_0));
+    const k::SplitX sx = k::SplitXView(split.p, static_cast<int>(n), static_cast<int>(cols),
+                                       static_cast<int>(2 * rows), type == kQ8_0);
     k::SplitRows(dx.as<float>(), cols, static_cast<int>(n), static_cast<int>(cols), nullptr, 0.0f, sx, nullptr);
     k::GemmJob g, u;
     g.w = HostMat(type, dg.as<uint8_t>(), rows, cols);
@@ -585,17 +587,17 @@ int32_t rpg_hip_attention(const float* q, const float* k, const float* v, int32_
   }, -1);
 }
 
-int32_t rpg_hip_split_layout(int32_t tokens, int32_t k, int32_t columns, int64_t* out) {
+int32_t rpg_hip_split_layout(int32_t tokens, int32_t k, int32_t columns, int32_t q8, int64_t* out) {
   return Guard([&]() -> int32_t {
     RPG_CHECK(tokens > 0 && k > 0 && columns > 0, "split_layout: empty shape");
     // (256: an address to tell the parts apart by, nothing is read there)
-    const k::SplitX x = k::SplitXView(reinterpret_cast<void*>(256), tokens, k, columns);
+    const k::SplitX x = k::SplitXView(reinterpret_cast<void*>(256), tokens, k, columns, q8 != 0);
     const auto at = [](const void* p) { return static_cast<int64_t>(reinterpret_cast<uintptr_t>(p)) - 256; };
     out[0] = at(x.hi);
     out[1] = at(x.inv_s + tokens);
     out[2] = at(x.part);
     out[3] = at(x.part + x.part_cap);
-    out[4] = static_cast<int64_t>(k::SplitXBytes(tokens, k, columns));
+    out[4] = static_cast<int64_t>(k::SplitXBytes(tokens, k, columns, q8 != 0));
     return 0;
   }, -1);
 }
@@ -639,7 +641,7 @@ int32_t rpg_hip_bench_matmul(uint32_t type, const uint8_t* w, int64_t rows, int6
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
-    DevBuf split(k::SplitXBytes(n_max, static_cast<int>(cols), static_cast<int>(rows)));
+    DevBuf split(k::SplitXBytes(n_max, static_cast<int>(cols), static_cast<int>(rows), type == kQ8_0));
     // a few tokens: time the decode paths, on tile-major copies
     bool want_tile = false;
     for (int i = 0; i < n_count; ++i) want_tile = want_tile || ns[i] <= k::FewTokenLimit();

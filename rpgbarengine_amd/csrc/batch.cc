@@ -53,7 +53,7 @@ void SessionBatch::Init() {
   work_stride_ = k::DecodeAttnBatchWorkFloats(c.n_heads, max_seq_all_);
   alloc(&work_, work_stride_);
   const int kmax = std::max({c.hidden, c.q_dim(), c.intermediate});
-  DeviceAlloc(&split_, k::SplitXBytes(B_, kmax, SplitColumns(c)));
+  DeviceAlloc(&split_, k::SplitXBytes(B_, kmax, SplitColumns(c), HasQ8(m_)));
   DeviceAlloc(&d_tok_, sizeof(int32_t) * B_);
   DeviceAlloc(&d_pos_, sizeof(int32_t) * B_);
   DeviceAlloc(&d_step_, sizeof(int32_t));
@@ -96,7 +96,7 @@ void SessionBatch::EnqueueStep(bool forced) {
   sampler_->Enqueue(logits_, c.vocab, d_pos_, 0, d_tok_, nullptr, stream_);
   if (forced) k::ForceTokens(d_tok_, B_, d_force_, d_drawn_, d_step_, out_cap_, stream_);
   k::GatherRows(m_.embd(), d_tok_, B_, x_, H, d_err_, stream_, d_out_, d_step_, out_cap_);
-  const FwdBufs b{x_, h_, q_, k_, v_, attn_, act_, gu_, split_, SplitColumns(c), stream_, side_, ev_fork_, ev_join_};
+  const FwdBufs b{x_, h_, q_, k_, v_, attn_, act_, gu_, split_, SplitColumns(c), HasQ8(m_), stream_, side_, ev_fork_, ev_join_};
   ForwardLayers(m_, b, B_, [&](int l, const LayerDev& w, const k::SplitPending* pend) {
     k::ApplyPending(pend[0], q_, c.q_dim(), c.q_dim(), stream_, k::kStore);
     k::ApplyPending(pend[1], k_, c.kv_dim(), c.kv_dim(), stream_, k::kStore);

@@ -23,11 +23,12 @@
 namespace rpg {
 
 // Device buffers (N tokens) and streams of one forward. split: SplitXBytes(N,
-// max K, split_cols) bytes; gu: [2][N][intermediate]; h: [N][max K].
+// max K, split_cols, split_q8) bytes; gu: [2][N][intermediate]; h: [N][max K].
 struct FwdBufs {
   float *x, *h, *q, *k, *v, *attn, *act, *gu;
   void* split;
   int split_cols;
+  bool split_q8;
   hipStream_t stream, side;
   hipEvent_t ev_fork, ev_join;
 };
@@ -35,6 +36,14 @@ struct FwdBufs {
 // Output columns of the widest GEMM launch that may split its K range (the
 // QKV projections; the gate+up pair never needs to): sizes the partials.
 inline int SplitColumns(const ModelConfig& c) { return std::max(c.hidden, c.q_dim() + 2 * c.kv_dim()); }
+
+// Whether a layer has Q8_0 projections (their GEMM takes more room for partials).
+inline bool HasQ8(const DeviceModel& m) {
+  for (const LayerDev& l : m.layers())
+    for (const k::MatRef* w : {&l.q, &l.k, &l.v, &l.o, &l.gate, &l.up, &l.down})
+      if (w->type == kQ8_0) return true;
+  return false;
+}
 
 // Every layer for N tokens whose embeddings are in b.x (row stride hidden).
 // attend(l, w, pend) computes layer l's attention from the raw projections b.q,
@@ -116,7 +125,7 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
       }
     }
     if (ng == 0) return;
-    const k::SplitX sx = k::SplitXView(b.split, N, K, b.split_cols);
+    const k::SplitX sx = k::SplitXView(b.split, N, K, b.split_cols, b.split_q8);
     k::SplitRowsAdd(const_cast<float*>(in), K, N, K, norm_w, c.rms_eps, sx, pend, stream);
     pend = k::SplitPending{};
     // one launch per weight type; a second type runs on the side stream
@@ -180,7 +189,7 @@ void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend)
     } else if (mma && k::QGemmSupports(w.gate) && k::QGemmSupports(w.up) && w.gate.type == w.up.type) {
       // one launch computes silu(gate) * up where the kernel allows, else
       // both products and the SwiGLU pass
-      const k::SplitX sx = k::SplitXView(b.split, N, H, b.split_cols);
+      const k::SplitX sx = k::SplitXView(b.split, N, H, b.split_cols, b.split_q8);
       k::SplitRowsAdd(x, H, N, H, w.ffn_norm, c.rms_eps, sx, pend, stream);
       pend = k::SplitPending{};
       if (!k::QGemmSwiGLU(sx, gj(w.gate, b.act, F, k::kStore).second, gj(w.up, nullptr, F, k::kStore).second,

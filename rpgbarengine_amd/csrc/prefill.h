@@ -46,10 +46,11 @@ struct SplitX {
   int32_t M = 0, K = 0;
 };
 // Bytes of a SplitX for up to M x K whose QGemm launches produce at most
-// n_max output columns in total (sizes the split-K partials).
-size_t SplitXBytes(int M, int K, int n_max);
-// Carve a SplitX out of `base` (SplitXBytes(M, K, n_max) bytes).
-SplitX SplitXView(void* base, int M, int K, int n_max);
+// n_max output columns in total (sizes the split-K partials); q8: Q8_0
+// matrices among them.
+size_t SplitXBytes(int M, int K, int n_max, bool q8);
+// Carve a SplitX out of `base` (SplitXBytes of the same figures).
+SplitX SplitXView(void* base, int M, int K, int n_max, bool q8);
 
 // x = X rows (stride ldx), or RMSNorm(x) * norm_w when norm_w != nullptr
 // (double sum of squares, float scale, (x * scale) * w, reference

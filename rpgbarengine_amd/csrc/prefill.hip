@@ -991,28 +991,28 @@ void SwiGLURows(const float* g, const float* u, float* y, int64_t n, hipStream_t
 
 namespace {
 // Floats of the split-K partials that the K-quants' splits plan with, and those
-// that the buffer holds: a tiled Q8_0 launch runs at most two rounds of partial
+// that the buffer holds: a tiled Q8_0 launch runs up to two rounds of partial
 // tiles (segments past the few-token matvec).
 int64_t PartFloats(int M, int n_max) { return static_cast<int64_t>(kGemmSplitMax) * M * n_max; }
-int64_t PartCap(int M, int n_max) {
-  return std::max<int64_t>(PartFloats(M, n_max), M > kMaxBatchTokens ? 512 * Q8TileTokens(M) * kQ8Rows : 0);
+int64_t PartCap(int M, int n_max, bool q8) {
+  return std::max<int64_t>(PartFloats(M, n_max), q8 && M > kMaxBatchTokens ? 512 * Q8TileTokens(M) * kQ8Rows : 0);
 }
 }  // namespace
 
-size_t SplitXBytes(int M, int K, int n_max) {
+size_t SplitXBytes(int M, int K, int n_max, bool q8) {
   const size_t big = static_cast<size_t>(M) * K * 2, small = static_cast<size_t>(M) * (K / 32) * 2;
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   return 2 * up(big) + 2 * up(small) + up(static_cast<size_t>(M) * 4) +
-         up(static_cast<size_t>(PartCap(M, n_max)) * 4);
+         up(static_cast<size_t>(PartCap(M, n_max, q8)) * 4);
 }
 
-SplitX SplitXView(void* base, int M, int K, int n_max) {
+SplitX SplitXView(void* base, int M, int K, int n_max, bool q8) {
   const size_t big = static_cast<size_t>(M) * K * 2, small = static_cast<size_t>(M) * (K / 32) * 2;
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   // The partial sums first, at an offset that does not depend on K: one
   // projection's stay there until the next one's operands are split (of another
   // width), each token's workgroup adding its own while others write operands.
-  uint8_t* p = static_cast<uint8_t*>(base) + up(static_cast<size_t>(PartCap(M, n_max)) * 4);
+  uint8_t* p = static_cast<uint8_t*>(base) + up(static_cast<size_t>(PartCap(M, n_max, q8)) * 4);
   SplitX s;
   s.part = static_cast<float*>(base);
   s.hi = p;
@@ -1021,7 +1021,7 @@ SplitX SplitXView(void* base, int M, int K, int n_max) {
   s.sum_lo = p + 2 * up(big) + up(small);
   s.inv_s = reinterpret_cast<float*>(p + 2 * up(big) + 2 * up(small));
   s.part_floats = PartFloats(M, n_max);
-  s.part_cap = PartCap(M, n_max);
+  s.part_cap = PartCap(M, n_max, q8);
   s.M = M;
   s.K = K;
   return s;

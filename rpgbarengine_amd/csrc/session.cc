@@ -266,7 +266,7 @@ void Session::EnsureScratch(int64_t tokens, int64_t logit_rows) {
     // (or the attention's images of a full cache, whatever was prefilled so
     // far: a conversation grown by short turns takes them too)
     const size_t split_bytes =
-        std::max(k::SplitXBytes(static_cast<int>(tokens), kmax, SplitColumns(c)),
+        std::max(k::SplitXBytes(static_cast<int>(tokens), kmax, SplitColumns(c), HasQ8(m_)),
                  sizeof(float) * static_cast<size_t>(k::AttnImageFloats(static_cast<int>(tokens), c.n_kv_heads, max_seq_)));
     DeviceAlloc(&split_, split_bytes);
     split_bytes_ = static_cast<int64_t>(split_bytes);
@@ -296,7 +296,7 @@ void Session::ForwardSegment(const int32_t* ids_dev, int64_t n, int64_t pos0, co
   RPG_CHECK(logit_rows <= logit_rows_cap_, "internal: %lld logits rows, capacity %lld", (long long)logit_rows,
             (long long)logit_rows_cap_);
   k::GatherRows(m_.embd(), ids_dev, N, x_, H, d_err_, stream_);
-  const FwdBufs b{x_, h_, q_, k_, v_, attn_, act_, gu_, split_, SplitColumns(c), stream_, side_, ev_fork_, ev_join_};
+  const FwdBufs b{x_, h_, q_, k_, v_, attn_, act_, gu_, split_, SplitColumns(c), HasQ8(m_), stream_, side_, ev_fork_, ev_join_};
   ForwardLayers(m_, b, N, [&](int l, const LayerDev& w, const k::SplitPending* pend) {
     k::QkvArgs qa;
     qa.q = q_;

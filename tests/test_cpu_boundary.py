@@ -129,14 +129,15 @@ def test_quantize_roundtrip_error(qtype):
 @pytest.mark.parametrize("hidden,q_dim,kv_dim,ffn", [(2560, 4096, 1024, 9728), (5120, 1024, 256, 512),
                                                      (5120, 2048, 256, 512), (2048, 2048, 1024, 6144)])
 @pytest.mark.parametrize("tokens", [2, 64, 65, 130, 512, 4096])
-def test_pending_sums_keep_clear_of_the_next_operands(hidden, q_dim, kv_dim, ffn, tokens):
+@pytest.mark.parametrize("q8", [False, True])
+def test_pending_sums_keep_clear_of_the_next_operands(hidden, q_dim, kv_dim, ffn, tokens, q8):
     """A projection's K parts stay in the buffer until the next operand split
     adds them, each token's workgroup its own, while others write the new
     operands: no projection's partial sums may lie where another's operands
     do, whatever the widths (the O projection of a model with hidden > q_dim
     splits K = q_dim, the gate and up after it K = hidden)."""
     columns = max(hidden, q_dim + 2 * kv_dim)
-    views = {k: eng.split_layout(tokens, k, columns) for k in {hidden, q_dim, ffn}}
+    views = {k: eng.split_layout(tokens, k, columns, q8) for k in {hidden, q_dim, ffn}}
     size = max(v[4] for v in views.values())
     for a in views.values():
         assert 0 <= a[0] < a[1] <= size and 0 <= a[2] < a[3] <= size
