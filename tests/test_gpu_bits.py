@@ -123,3 +123,17 @@ def test_conversation_bits(gguf_factory):
             x.prefill(ids(100 + n))
         got, _ = eng.generate_batch(sessions, 16, 0.2, 0, 0.95, [9 + i for i in range(n)])
         assert (_crc(got), _crc(np.stack([x.prefill(ids(3)) for x in sessions]))) == (reply, after)
+
+
+@pytest.mark.parametrize("mix", ["q4_k_m", "q8_0"])
+def test_bits_do_not_depend_on_a_sessions_past(gguf_factory, mix):
+    """The same turns give the same logits in a session that only ever took
+    short segments and in one whose scratch a long segment has grown."""
+    model = eng.Model(gguf_factory("small", mix), max_pos=2048)
+    rng = np.random.default_rng(8)
+    turns = [rng.integers(0, 4096, n, dtype=np.int32) for n in (70, 90, 33, 128, 100, 2, 81)]
+    short, grown = model.session(1500), model.session(1500)
+    grown.prefill(rng.integers(0, 4096, 1400, dtype=np.int32))
+    grown.set_len(0)
+    for t in turns:
+        assert np.array_equal(short.prefill(t).view(np.uint32), grown.prefill(t).view(np.uint32))

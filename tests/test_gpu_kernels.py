@@ -142,7 +142,11 @@ def test_tiled_gemm_ragged_shapes(qtype, k, rows, m):
 # it in theirs.
 @pytest.mark.parametrize("qtype,k,rows,m", [(synth.Q8_0, 2560, 300, 130), (synth.Q8_0, 256, 1, 100),
                                             (synth.Q8_0, 9728, 257, 129), (synth.Q6_K, 9728, 257, 129),
-                                            (synth.Q4_K, 9728, 513, 97)])
+                                            (synth.Q4_K, 9728, 513, 97),
+                                            # tiles of 128 tokens, the last with 65, 1 and 66 of them
+                                            (synth.Q8_0, 2304, 641, 321), (synth.Q8_0, 9728, 257, 385),
+                                            (synth.Q8_0, 512, 300, 450), (synth.Q6_K, 2304, 641, 385),
+                                            (synth.Q4_K, 2304, 641, 385)])
 def test_tiled_gemm_parts(qtype, k, rows, m):
     w32 = synth.gaussian(41, k + rows + qtype, rows * k, 0.02).reshape(rows, k)
     raw = synth.quantize(qtype, w32)
