@@ -128,12 +128,13 @@ def test_conversation_bits(gguf_factory):
 @pytest.mark.parametrize("mix", ["q4_k_m", "q8_0"])
 def test_bits_do_not_depend_on_a_sessions_past(gguf_factory, mix):
     """The same turns give the same logits in a session that only ever took
-    short segments and in one whose scratch a long segment has grown."""
-    model = eng.Model(gguf_factory("small", mix), max_pos=2048)
+    short segments and in one whose scratch a long segment has grown (8 KV
+    heads, to a history whose key images are some 30 MB)."""
+    model = eng.Model(gguf_factory("tiny", mix, n_heads=16, n_kv_heads=8), max_pos=4096)
     rng = np.random.default_rng(8)
-    turns = [rng.integers(0, 4096, n, dtype=np.int32) for n in (70, 90, 33, 128, 100, 2, 81)]
-    short, grown = model.session(1500), model.session(1500)
-    grown.prefill(rng.integers(0, 4096, 1400, dtype=np.int32))
+    turns = [rng.integers(0, 1024, n, dtype=np.int32) for n in [100] * 36 + [70, 33, 128, 2, 81]]
+    short, grown = model.session(4096), model.session(4096)
+    grown.prefill(rng.integers(0, 1024, 4096, dtype=np.int32))
     grown.set_len(0)
     for t in turns:
         assert np.array_equal(short.prefill(t).view(np.uint32), grown.prefill(t).view(np.uint32))
