@@ -159,8 +159,8 @@ constexpr int kQB = 16;        // queries per query tile (one tile per workgroup
 // launch of their own, instead of by every query block that walks them: the
 // conversion took more issue slots than the products (~400 VALU instructions
 // per wave and step of 64 keys against 48 MFMAs). Per layer, us, before / after
-// (conversion included): 3999 tokens of the 1.7B shape 477 / 374, 512 of the 4B
-// 36 / 32, 203 behind 1500 60 / 55; at fewer query blocks the launch (5 - 10 us)
+// (conversion included): 3999 tokens of the 1.7B shape 477 / 407, 512 of the 4B
+// 38 / 36, 203 behind 1500 106 / 82; at fewer query blocks the launch (7 - 10 us)
 // costs what it saves.
 constexpr int kImageQueryBlocks = 6;
 constexpr int kWideQueries = 1024;  // segments at least this long take two query tiles per workgroup (G <= 2)

@@ -48,8 +48,8 @@ inline bool HasQ8(const DeviceModel& m) {
 // Every layer for N tokens whose embeddings are in b.x (row stride hidden).
 // attend(l, w, pend) computes layer l's attention from the raw projections b.q,
 // b.k, b.v into b.attn (and writes the cache); where pend[i].part is set,
-// projection i is still in pending partial sums instead of its buffer. On return b.x holds the final
-// residual stream, every pending split-K sum applied.
+// projection i is still in pending partial sums instead of its buffer. On
+// return b.x holds the final residual stream, every pending split-K sum applied.
 template <typename Attend>
 void ForwardLayers(const DeviceModel& m, const FwdBufs& b, int N, Attend attend) {
   const ModelConfig& c = m.config();

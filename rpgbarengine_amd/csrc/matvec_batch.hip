@@ -79,10 +79,11 @@ typedef float F4 __attribute__((ext_vector_type(4)));
 typedef float F2 __attribute__((ext_vector_type(2)));
 
 constexpr int kLdsBudget = 150 * 1024;  // staged tokens + per-group sums of one workgroup
-// Segments of up to 64 tokens take the few-token launches. A wide projection of
-// some 40 tokens is faster on the GEMM (4B gate+up of 37 tokens 53 us against
-// 35), whose hi + lo operands hold 22 bits below a token's largest input,
-// though, against 22 below its 32-group's here, and 30 of a Q8_0 launch.
+// Segments of up to 64 tokens take the few-token launches, faster than the
+// 32-token GEMMs on every 1.7B / 4B shape. A GEMM of 64-token tiles can be
+// faster from some 40 tokens on (1.7B Q8_0 gate+up of 48 tokens 44 us against
+// 37), but its hi + lo operands hold 22 bits below a token's largest input,
+// where the ones here hold 22 below its 32-group's, and 30 in a Q8_0 launch.
 constexpr int kFewTokensDefault = 64;
 constexpr int kRecBytes = 96;       // digit rows of one token and group (three digits)
 constexpr int kRecBytes4 = 128;     // the same with four digits (Q8_0 launches)

@@ -2,12 +2,14 @@
 //
 // Y[t][n] = sum_k X[t][k] * W[n][k] for a segment of M tokens and a raw GGUF
 // weight matrix W (Q4_K, Q6_K or Q8_0). The product runs on
-// v_mfma_f32_16x16x32_f16 with operands that make it exact up to fp32
+// v_mfma_f32_16x16x32_f16 (prefill.hip) or v_mfma_f32_32x32x16_f16
+// (gemm_tiled.hip, gemm_q8.hip) with operands that make it exact up to fp32
 // accumulation:
 //  * W side: the integer quants times their integer sub-block scales, which
 //    are small enough to be exact in f16 (Q4_K: q*sc <= 945; Q6_K: (q-32)*sc
-//    split into 16*(q-32)*floor(sc/16) and (q-32)*(sc mod 16); Q8_0: q);
-//    the fp16 block scales d (and dmin) are applied in fp32 once per block.
+//    split into 16*(q-32)*floor(sc/16) and (q-32)*(sc mod 16), in the tiled
+//    kernel q - 32, its products scaled by d*sc in fp32; Q8_0: q); the fp16
+//    block scales d (and dmin) are applied in fp32 once per block.
 //  * X side: each token row scaled by a power of two s so that max|x*s| lies
 //    in [2^14, 2^15), then split x*s = hi + lo into two f16 (22 significant
 //    bits), both multiplied into the same accumulator.
@@ -96,10 +98,10 @@ void SwiGLURows(const float* g, const float* u, float* y, int64_t n, hipStream_t
 // Tiled Q4_K / Q6_K GEMM (gemm_tiled.hip): 128 tokens x 128 weight rows per
 // workgroup, each step's weights unpacked once into LDS. QGemm and QGemmSwiGLU
 // take it for segments of at least kTiledMinTokens tokens.
-// A kernel of 64 x 64 wave tiles with weights unpacked in registers, in the
-// form of gemm_q8.hip, ran these too and faster (4B 512 tokens 14.1 -> 12.7 ms,
-// 203 behind 1500 12.9 -> 9.5), closer to float64, but in another order of sums:
-// see QGemm's part_floats, and the replies that a seed gives.
+// The form of gemm_q8.hip (64 x 64 wave tiles, weights unpacked in registers)
+// was faster for these too (4B 512 tokens 14.1 -> 12.7 ms) and closer to
+// float64, but another order of sums gives another reply to a seed wherever a
+// draw falls between two roundings.
 constexpr int kTiledTokens = 128;
 constexpr int kTiledRows = 128;
 constexpr int kTiledMinTokens = 96;
